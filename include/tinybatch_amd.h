@@ -249,6 +249,42 @@ int32_t tb_paged_prefill(const void* q, int64_t q_row_stride, void* pool, int64_
                          const void* k_new, int64_t k_row_stride, const void* v_new, int64_t v_row_stride,
                          const float* rope_cos, const float* rope_sin, int32_t rope_max_position,
                          hipStream_t stream);
+/* K2 for prefill rows of any context (reference src/tinybatch/model.py:130-147), column
+ * tiles: fp16 / bf16, head_dim 64 or 128, block_size a power of two >= 16, any number of
+ * query heads per kv head (TB_ERR_UNSUPPORTED otherwise: use tb_paged_attention's tiles).
+ * The rows it serves must not also be given to tb_paged_attention as work items or tiles.
+ * The K/V of the step's new rows must already be in the pool (append first).
+ *   work: tb_build_prefill_columns_work's list (device memory, 16-byte aligned), num_work
+ *     entries of 8 int32; row_part_offsets [num_rows + 1]: as tb_paged_attention takes it,
+ *     with ceil(row_ctx / partition_tokens) partitions for every row served here;
+ *   split_rows [num_split_rows][4] (row, first partial slot, count, 0): the rows whose
+ *     partials this call merges at its end; 0 leaves them to a tb_paged_attention call that
+ *     follows on the same stream with the same workspace;
+ *   workspace (when max_parts_per_row > 1): as tb_paged_attention; NULL: the static scratch
+ *     of tb_paged_attention_noalloc (TB_ERR_SCRATCH past its size; overlapping calls race).
+ * q, out, strides, scale, dtype, rope: as tb_paged_attention. */
+int32_t tb_paged_prefill_columns(const void* q, int64_t q_row_stride, const void* pool, int64_t num_blocks,
+                                 void* out, int64_t out_row_stride, const int32_t* block_tables,
+                                 int32_t max_blocks_per_seq, const int32_t* work, int32_t num_work,
+                                 const int32_t* row_part_offsets, int32_t num_rows,
+                                 const int32_t* split_rows, int32_t num_split_rows,
+                                 int32_t max_parts_per_row, int32_t total_partitions, int32_t num_heads,
+                                 int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale,
+                                 int32_t dtype, void* workspace, size_t workspace_bytes,
+                                 const float* rope_cos, const float* rope_sin, int32_t rope_max_position,
+                                 hipStream_t stream);
+/* The partition length (positions, a multiple of 64) for a step's sequences of new_rows new
+ * rows from position pos0 on a GPU of num_cus CUs: longer than every context unless the
+ * step has too few rows to keep the CUs busy. Negative: a status code. */
+int32_t tb_prefill_columns_partition(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs,
+                                     int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t num_cus);
+/* The work list (host, no device call): *count entries of 8 int32 into work (work NULL: the
+ * count alone). Entry g is meant for XCD g % num_xcds (1: placement unknown). */
+int32_t tb_build_prefill_columns_work(const int32_t* first_row, const int32_t* seq_index, const int32_t* pos0,
+                                      const int32_t* new_rows, int32_t num_seqs, int32_t num_heads,
+                                      int32_t num_kv_heads, int32_t partition_tokens, int32_t num_xcds,
+                                      int32_t num_cus, int32_t* work, int32_t capacity, int32_t* count);
+
 /* The longest context (positions) and the most query heads per kv head
  * tb_paged_prefill serves at a head dim (0: none). */
 int32_t tb_prefill_stream_max_context(int32_t head_dim);

@@ -1,0 +1,58 @@
+"""tb_build_prefill_columns_work (host code, no GPU): every (query row, head, position) a
+sequence's rows may see is covered by exactly one entry; padding entries have no rows; the
+partition rule keeps rows whole when the step fills the GPU and never asks for more
+scratch than the tiles did, past the static scratch."""
+import numpy as np
+import pytest
+
+from tinybatch_amd.metadata import (TILE_PARTITION, ColumnsRoute, build_columns_work, build_step_metadata,
+                                    columns_partition)
+
+
+def covered(first, pos0, rows, hq, hkv, work, part):
+    """How often each (row, head) meets each partition it has positions in."""
+    rep = hq // hkv
+    seen = [np.zeros((n, hq, -(-(p + n) // part)), dtype=int) for p, n in zip(pos0, rows)]
+    for r0, seq, p0, n, col0, kvh, p, pc in work.tolist():
+        if n == 0:
+            continue
+        assert (r0, p0, n, pc) == (first[seq], pos0[seq], rows[seq], part // 64)
+        for col in range(col0, min(col0 + 128, n * rep)):
+            seen[seq][col // rep, kvh * rep + col % rep, p] += 1
+    for s, p0, n in zip(seen, pos0, rows):
+        for r in range(n):
+            mine = -(-(p0 + r + 1) // part)
+            assert (s[r, :, :mine] == 1).all() and (s[r, :, mine:] <= 1).all()
+
+
+@pytest.mark.parametrize("hq,hkv", [(14, 2), (32, 8), (5, 1), (4, 4)])
+@pytest.mark.parametrize("xcds", [1, 8])
+@pytest.mark.parametrize("part", [64, 512, 1 << 20])
+def test_every_row_head_and_partition_once(hq, hkv, xcds, part):
+    rows, pos0 = [16, 19, 64, 129, 300], [0, 45, 1000, 63, 2]
+    first = np.concatenate([[0], np.cumsum(rows)[:-1]]).tolist()
+    work = build_columns_work(first, range(5), pos0, rows, part, ColumnsRoute(hq, hkv, 64, xcds, 256))
+    assert len(work) % xcds == 0
+    covered(first, pos0, rows, hq, hkv, work, part)
+
+
+def test_partitions():
+    r = ColumnsRoute(14, 2, 64, 8, 256)
+    assert columns_partition([0] * 4, [3251, 1746, 3738, 2168], r) > 3738         # enough rows: none split
+    p = columns_partition([3000] * 4, [20] * 4, r)
+    assert p % 64 == 0 and p <= TILE_PARTITION
+    p = columns_partition([9000], [1500], r)                                    # the scratch bound
+    assert p == TILE_PARTITION
+    with pytest.raises(RuntimeError):
+        columns_partition([0], [0], r)
+
+
+def test_metadata_counts_partitions_of_the_columns():
+    r = ColumnsRoute(14, 2, 64, 8, 256)
+    m = build_step_metadata(list(range(2000, 2040)) + [99], [(0, 40), (40, 41)], [list(range(128)), [200] * 7],
+                            [2040, 100], block_size=16, num_blocks=256, partition_tokens=256, rows_per_item=2,
+                            tile_prefill=True, columns_route=r)
+    part = columns_partition([2000], [40], r)
+    assert m.num_columns_work and m.num_prefill_tiles == 0 and m.num_work_items == 1
+    assert np.diff(m.row_part_off_np).tolist() == [-(-(2001 + i) // part) for i in range(40)] + [1]
+    assert m.split_rows_np[:, 0].tolist() == list(range(40))

@@ -98,6 +98,16 @@ SIGNATURES = {
         c_i32, c_i32, c_i32, c_i32, c_f32, c_i32,   # heads, kv heads, head_dim, block_size, scale, dtype
         c_vp, c_i64, c_vp, c_i64,                # k_new, k stride, v_new, v stride (fused append, may be NULL)
         c_vp, c_vp, c_i32, c_vp]),               # rope cos, sin, max position, stream
+    "tb_paged_prefill_columns": (c_i32, [
+        c_vp, c_i64, c_vp, c_i64, c_vp, c_i64,   # q, q stride, pool, num_blocks, out, out stride
+        c_vp, c_i32, c_vp, c_i32,                # block tables, max_nb, work, num_work
+        c_vp, c_i32, c_vp, c_i32, c_i32, c_i32,  # row_part_offsets, rows, split rows, count, max parts, total partitions
+        c_i32, c_i32, c_i32, c_i32, c_f32, c_i32,   # heads, kv heads, head_dim, block_size, scale, dtype
+        c_vp, c_sz,                              # workspace, bytes
+        c_vp, c_vp, c_i32, c_vp]),               # rope cos, sin, max position, stream
+    "tb_prefill_columns_partition": (c_i32, [c_vp, c_vp, c_i32, c_i32, c_i32, c_i32, c_i32]),
+    "tb_build_prefill_columns_work": (c_i32, [c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32,
+                                              c_vp, c_i32, c_vp]),
     "tb_prefill_stream_max_context": (c_i32, [c_i32]),
     "tb_prefill_stream_max_group": (c_i32, [c_i32]),
     "tb_prefill_work_count": (c_i32, [c_vp, c_i32, c_i32]),

@@ -1188,6 +1188,25 @@ static void launch_16bit(const attn_args& a, bool d64, int num_work, int num_til
   }
 }
 
+void combine_split_rows(int32_t dtype, int32_t head_dim, int32_t num_heads, void* out, int64_t out_row_bytes,
+                        const int32_t* split_rows, int32_t num_split_rows, float* ws_acc, float* ws_ml,
+                        hipStream_t stream) {
+  attn_args a{};
+  a.out = (char*)out;
+  a.out_row_bytes = out_row_bytes;
+  a.split_rows = reinterpret_cast<const int4*>(split_rows);
+  a.ws_acc = ws_acc;
+  a.ws_ml = ws_ml;
+  a.num_heads = num_heads;
+  const bool d64 = head_dim == 64;
+  if (dtype == TB_DTYPE_F16)
+    d64 ? launch_combine<f16_t, 64>(a, num_split_rows, stream) : launch_combine<f16_t, 128>(a, num_split_rows, stream);
+  else if (dtype == TB_DTYPE_BF16)
+    d64 ? launch_combine<bf16_t, 64>(a, num_split_rows, stream) : launch_combine<bf16_t, 128>(a, num_split_rows, stream);
+  else
+    d64 ? launch_combine<f32_t, 64>(a, num_split_rows, stream) : launch_combine<f32_t, 128>(a, num_split_rows, stream);
+}
+
 static int largest_divisor_upto(int rep, int cap) {
   for (int t = cap; t >= 1; --t)
     if (rep % t == 0) return t;
@@ -1373,7 +1392,7 @@ constexpr int MAX_DEVICES = 64;
 static std::atomic<void*> scratch_ptr[MAX_DEVICES];
 static std::mutex scratch_mu;
 
-static int32_t scratch_address(hipStream_t stream, void** ptr) {
+int32_t noalloc_scratch(hipStream_t stream, void** ptr) {
   int dev = -1;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return TB_ERR_LAUNCH;
   if (stream != nullptr) {   // the stream must belong to the current device, whose copy is used
@@ -1441,7 +1460,7 @@ extern "C" int32_t tb_paged_attention_noalloc(const void* q, int64_t q_row_strid
   if (max_parts_per_row > 1) {   // partials are only written for rows of more than one partition
     const size_t need = tb_paged_attention_workspace_bytes(total_partitions, num_heads, head_dim);
     if (need > (size_t)TB_NOALLOC_SCRATCH_BYTES) return TB_ERR_SCRATCH;
-    const int32_t st = tb::scratch_address(stream, &ws);
+    const int32_t st = tb::noalloc_scratch(stream, &ws);
     if (st != TB_OK) return st;
     ws_bytes = TB_NOALLOC_SCRATCH_BYTES;
   }

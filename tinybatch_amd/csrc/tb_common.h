@@ -272,6 +272,14 @@ struct rope_tables {
   }
 };
 
+// Host helpers shared by the entry points (tb_attention.hip).
+// The log-sum-exp merge of split rows' partials (records (row, first slot, count, 0)) into out.
+void combine_split_rows(int32_t dtype, int32_t head_dim, int32_t num_heads, void* out, int64_t out_row_bytes,
+                        const int32_t* split_rows, int32_t num_split_rows, float* ws_acc, float* ws_ml,
+                        hipStream_t stream);
+// The device address of the static scratch (TB_NOALLOC_SCRATCH_BYTES) of the stream's GPU.
+int32_t noalloc_scratch(hipStream_t stream, void** ptr);
+
 }  // namespace tb
 
 // Status helpers shared by the C entry points.

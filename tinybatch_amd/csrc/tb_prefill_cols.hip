@@ -1,0 +1,575 @@
+// K2 for prefill rows of any context, column tiles (fp16 / bf16): the attention of a
+// sequence's new rows over its whole context (reference src/tinybatch/model.py:130-147:
+// gather, repeat_interleave, the mask of model.py:139-146 and SDPA).
+//
+// Work: the new rows of a sequence and the rep query heads of a kv head make
+// n * rep columns, column = row * rep + head; a workgroup takes NW * 32 consecutive
+// columns (every head of NW * 32 / rep rows), wave w its columns 32 w .. 32 w + 31. So all
+// of a workgroup's columns read the same K/V rows, whatever rep is, with no padded
+// columns but the sequence's last ones, and its rows lie close together, so that few
+// scores past the diagonal are computed. The workgroup walks its positions in chunks of
+// 64.
+//
+// Loads. A chunk's K and V rows go to LDS by direct global->LDS loads (1 KiB of
+// consecutive pool bytes per instruction) through a ring of two chunks: the next chunk is
+// issued as a chunk's computation starts, so one wait (for the wave's own loads) and one
+// barrier per chunk are all the synchronisation. Rows past the workgroup's last position
+// repeat the last one: their scores are masked.
+//
+// Math per chunk, the wave's 32 columns as the 32 MFMA columns:
+//   S^T[pos][col] = K[pos][:] . q[col][:]         v_mfma_f32_32x32x16, A = K rows (LDS)
+//   O^T[d][col]  += V^T[d][pos] . P^T[pos][col]   v_mfma_f32_32x32x16, A = V^T (LDS
+//                                                  transpose reads), B = the S^T registers
+// so that each K or V value read from LDS meets 32 columns, and the online softmax state
+// of column l % 32 lives in lanes l and l ^ 32.
+//
+// What bounds it and what it measured (bf16, us per layer, against the 64-row tiles of
+// tb_attention.hip): three prompts of 5300..7333 tokens at 32 / 8 heads of 128: 1090 us =
+// 994 TFLOP/s against 3260 + 290 for the merge of split rows; four of 1746..3738 at 14 / 2
+// heads of 64: 86 us = 670 TFLOP/s against 122 + 14. (A plain 8192^3 library product
+// reaches 1232 TFLOP/s on this card.) At head dim 128 a chunk takes a SIMD's two waves
+// 3800 cycles, 2050 of them MFMA, at a shader clock that falls to 1.7 to 2.0 GHz; at 64
+// the softmax (32 exponentials, FMAs and packs a chunk) and its issue bound it. Measured
+// and not kept: 256 columns in eight waves (one workgroup per CU at head dim 128, whose
+// start and end, 9 us of 65, nothing then overlaps: 1140 us); the two waves of a SIMD
+// held half a chunk apart by barriers (930 against 911 us on six prompts of 4096); the next
+// chunk's scores computed under this chunk's exponentials (spills at head dim 128); a
+// chunk's loads spread between its products (the same); row sums on the matrix unit (5%
+// slower at head dim 64).
+#include <algorithm>
+#include <vector>
+
+#include "tb_stream.h"
+
+namespace tb {
+
+typedef float float16_t __attribute__((ext_vector_type(16)));
+
+template <typename Tag>
+struct cmath;
+template <>
+struct cmath<f16_t> {
+  typedef shalf8_t vec8_t;
+  static __device__ __forceinline__ float16_t mfma(su32x4_t a, su32x4_t b, float16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(shalf8_t, a), __builtin_bit_cast(shalf8_t, b), c,
+                                                   0, 0, 0);
+  }
+  // acc + the two halves of p (times one each)
+  static __device__ __forceinline__ float add2(uint32_t p, uint32_t ones, float acc) {
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, p), __builtin_bit_cast(half2_t, ones), acc, false);
+  }
+  static constexpr uint32_t ONES = 0x3C003C00u;
+};
+template <>
+struct cmath<bf16_t> {
+  typedef sbf168_t vec8_t;
+  static __device__ __forceinline__ float16_t mfma(su32x4_t a, su32x4_t b, float16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(sbf168_t, a), __builtin_bit_cast(sbf168_t, b),
+                                                    c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ float add2(uint32_t p, uint32_t ones, float acc) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf162_t, p), __builtin_bit_cast(bf162_t, ones), acc, false);
+  }
+  static constexpr uint32_t ONES = 0x3F803F80u;
+};
+
+struct cols_args {
+  const char* q;               // [T][Hq][D] rows of the step
+  int64_t q_row_bytes;
+  const char* pool;            // [NB][2][Hkv][BS][D]
+  int64_t num_blocks;
+  char* out;                   // [T][Hq*D]
+  int64_t out_row_bytes;
+  const int32_t* block_tables; // [B][max_nb]
+  int32_t max_nb;
+  const int4* work;            // two per workgroup: (row0, seq, pos0, nrows), (first column, kv head, part, part chunks)
+  const int32_t* row_part_off; // partial slots of the step's rows
+  float* ws_acc;               // [parts][Hq][D]
+  float* ws_ml;                // [parts][Hq][2]
+  int32_t num_heads, num_kv_heads, rep;
+  int32_t log2_bs;             // block size: a power of two >= 16
+  float scale_log2e;
+  rope_tables rope;
+};
+
+template <int D>
+struct cshape {
+  static constexpr int NW = 4;                  // waves per workgroup
+  static constexpr int RB = 2 * D;              // bytes per K or V row
+  static constexpr int TB = 16 * RB;            // bytes of a 16-position K (or V) tile
+  static constexpr int CK = 64;                 // positions per chunk
+  static constexpr int HALF = CK * RB;          // bytes of a chunk's K (or V) rows
+  static constexpr int SLOT = 2 * HALF;         // K then V
+  static constexpr int RING = 2;              // chunks in LDS: two or three workgroups on a CU
+  static constexpr int VCOLS = RB / 16;         // 16-byte pieces per row
+  static constexpr int RPL = 64 / VCOLS;        // rows per direct load
+  static constexpr int TLD = TB / 1024;         // direct loads per 16-position tile
+  static constexpr int KS = D / 16;             // q.k slices of 16 dims
+  static constexpr int NB = D / 32;             // O^T blocks of 32 dims
+  static constexpr int COLS = 32 * NW;          // columns per workgroup
+  static_assert(CK == 16 * NW, "wave w loads tile w of a chunk");
+  // K row r keeps its 16-byte piece c in slot c ^ kswz(r): the 16 rows that 16 lanes of an
+  // operand read touch then cover all 64 banks (rows 2 apart share banks at D = 64)
+  static __device__ __forceinline__ int kswz(int r) { return D == 64 ? (r & 7) ^ ((r >> 3) & 1) : r & 15; }
+  // V row r keeps piece c in slot c ^ vswz(r): the transpose reads of 32 lanes (4 rows x
+  // 64 bytes) cover all 64 banks
+  static __device__ __forceinline__ int vswz(int r) {
+    return D == 64 ? 2 * (r & 3) : (0xCA60 >> (4 * (r & 3))) & 15;
+  }
+};
+
+template <typename Tag, int D>
+__global__ __launch_bounds__(64 * cshape<D>::NW, 2) void paged_prefill_columns_kernel(const cols_args a) {
+  using S = cshape<D>;
+  using M = cmath<Tag>;
+  typedef typename smath<Tag>::scalar_t scalar_t;
+  constexpr int RB = S::RB, TB = S::TB, CK = S::CK, KS = S::KS, NB = S::NB;
+  __shared__ __align__(1024) char lds[S::RING * S::SLOT];
+
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, lcol = lane & 31, half = lane >> 5;
+  const int4 w0 = a.work[2 * blockIdx.x], w1 = a.work[2 * blockIdx.x + 1];
+  const int row0 = w0.x, seq = w0.y, pos0 = w0.z, nrows = w0.w;
+  if (nrows == 0) return;                       // a padding entry (whole workgroup)
+  const int col0 = w1.x, kvh = w1.y, part = w1.z, part_chunks = w1.w;
+  const int rep = a.rep, ncols = nrows * rep;
+
+  // this lane's column: query row my_row of the sequence's new rows, head hd
+  const int col = col0 + 32 * wave + lcol;
+  const bool mine = col < ncols;
+  const int ccol = mine ? col : ncols - 1;
+  const int my_row = ccol / rep, hd = kvh * rep + ccol - my_row * rep;
+  const int my_pos = pos0 + my_row;             // sees positions 0 .. my_pos
+  // wave-uniform: the positions of the wave's first and last column, the workgroup's positions
+  const int wcol = min(col0 + 32 * wave, ncols - 1);
+  const bool wave_busy = col0 + 32 * wave < ncols;
+  const int wave_first = pos0 + wcol / rep;
+  const int wave_last = pos0 + min(col0 + 32 * wave + 31, ncols - 1) / rep;
+  const int limit = pos0 + min(col0 + S::COLS - 1, ncols - 1) / rep + 1;
+  const int c_begin = part * part_chunks;
+  const int c_end = min(c_begin + part_chunks, (limit + CK - 1) / CK);
+
+  // ---- q (B operand: lane holds dims 16 s + 8 half .. of its column) ----
+  vec16 qv[KS];
+  {
+    const char* qrow = a.q + (int64_t)(row0 + my_row) * a.q_row_bytes + (int64_t)hd * RB + 16 * half;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qv[s] = ld16(qrow + 32 * s);
+  }
+
+  // ---- direct loads: pair i of this wave is tile lt[i] of the chunk, K or V ----
+  const int64_t head_bytes = ((int64_t)1 << a.log2_bs) * RB;     // one kv head's K (or V) rows of a block
+  const int64_t blk_bytes = 2 * (int64_t)a.num_kv_heads * head_bytes;
+  const int64_t v_off = a.num_kv_heads * head_bytes;
+  const int sub_mask = (1 << (a.log2_bs - 4)) - 1;                // 16-position tiles per block - 1
+  const int32_t* const table = a.block_tables + (int64_t)seq * a.max_nb;
+  const char* const pool_kvh = a.pool + kvh * head_bytes;
+  const int last_tile = (limit - 1) >> 4;
+  const int lt = wave;                          // the tile of a chunk this wave loads, K and V
+  const int lrow = lane / S::VCOLS, lpiece = lane % S::VCOLS;
+  // lane j: the block of this wave's tile in chunk id0 + j
+  int id0 = c_begin;
+  auto load_ids = [&](int c) {
+    const int t = min(4 * (c + lane) + lt, last_tile);
+    int b = table[(t << 4) >> a.log2_bs];
+    return (b < 0 || b >= a.num_blocks) ? 0 : b;   // host validates; stay inside the pool
+  };
+  int ids = load_ids(id0);
+  auto issue = [&](int c, int slot) {
+    if (c - id0 >= 64) {                        // uniform, once per 64 chunks
+      id0 = c;
+      ids = load_ids(id0);
+    }
+    const int t = min(4 * c + lt, last_tile);
+    const int rmax = limit - 1 - 16 * t;        // rows past it repeat the workgroup's last position
+    const int64_t b = __builtin_amdgcn_readlane(ids, c - id0);
+    const char* const base = pool_kvh + b * blk_bytes + (int64_t)(t & sub_mask) * TB;
+    char* const dst = lds + slot * S::SLOT + lt * TB;
+#pragma unroll
+    for (int i = 0; i < S::TLD; ++i) {
+      const int r = S::RPL * i + lrow;
+      const uint32_t row = (uint32_t)(min(r, rmax) * RB);
+      s_dma16_l2(row + 16 * (lpiece ^ S::kswz(r)), base, dst + 1024 * i);
+      s_dma16_l2(row + 16 * (lpiece ^ S::vswz(r)), base + v_off, dst + S::HALF + 1024 * i);
+    }
+  };
+  asm volatile("" : "+v"(ids));                 // the block ids have landed: no wait inside the loop
+  if (c_begin < c_end) issue(c_begin, 0);
+
+  // ---- q rotated (RoPE at the column's position), complete here ----
+  if (a.rope.cos) {
+    const int64_t r = a.rope.row(my_pos, D / 2) + 8 * half;
+#pragma unroll
+    for (int s = 0; s < KS / 2; ++s)            // slices s and s + KS/2 pair (dims i and i + D/2)
+      rope_pair<scalar_t>(qv[s], qv[s + KS / 2], a.rope.cos + r + 16 * s, a.rope.sin + r + 16 * s);
+  }
+  su32x4_t q[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    q[s] = __builtin_bit_cast(su32x4_t, qv[s]);
+    asm volatile("" : "+v"(q[s]));
+  }
+
+  uint32_t ones = M::ONES;                      // in a register: as a literal the bf16 dot product read it wrong
+  asm volatile("" : "+v"(ones));
+  float m = -INFINITY, l = 0.f;                 // reference max (scaled, base-2) and this lane's share of the sum
+  float16_t acc[NB];                            // O^T[32 b + 8 (r / 4) + 4 half + r % 4][col]
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
+
+  // operand addresses of this lane in a ring slot
+  uint32_t ka[KS], va[NB];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) ka[s] = (uint32_t)(lcol * RB + 16 * ((2 * s + half) ^ S::kswz(lcol)));
+  {
+    const int li = lane & 15, rv = 4 * half + (li >> 2);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int c = 4 * b + 2 * ((lane >> 4) & 1) + ((li & 3) >> 1);
+      va[b] = (uint32_t)(S::HALF + rv * RB + 16 * (c ^ S::vswz(rv)) + 8 * (li & 1));
+    }
+  }
+  const float sl2e = a.scale_log2e;
+
+  float16_t sc[2];                              // S^T: positions 64 c + 32 t + 8 (r / 4) + 4 half + r % 4 of column lcol
+  su32x4_t pb[4];                               // P of a chunk: B operands of 16 positions each
+  // S^T = K.q of the chunk in a slot
+  auto scores = [&](int slot) {
+    const char* const base = lds + slot * S::SLOT;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sc[t][r] = 0.f;
+    // operands read KG slices ahead of their products, pinned by the scheduling barriers:
+    // left to itself the compiler keeps one slice in flight and every product waits out
+    // an LDS latency
+    constexpr int KG = 2;
+    su32x4_t kf[2][KG][2];
+    auto read = [&](int g) {
+#pragma unroll
+      for (int i = 0; i < KG; ++i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          kf[g & 1][i][t] = *reinterpret_cast<const su32x4_t*>(base + ka[KG * g + i] + 32 * t * RB);
+    };
+    read(0);
+#pragma unroll
+    for (int g = 0; g < KS / KG; ++g) {
+      if (g + 1 < KS / KG) read(g + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < KG; ++i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) sc[t] = M::mfma(kf[g & 1][i][t], q[KG * g + i], sc[t]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // the online softmax of chunk c: sc -> pb, and the state's rescale
+  auto softmax = [&](int c) {
+    if (CK * c + CK - 1 > wave_first) {         // the chunk crosses the diagonal of some column
+      // kept a branch (most chunks skip it): folded into selects it cost every chunk 96
+      // vector instructions beside the 150 it needs
+      asm volatile("");
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (CK * c + 32 * t + 8 * (r >> 2) + 4 * half + (r & 3) > my_pos) sc[t][r] = -INFINITY;
+    }
+    float cm = max_f32(sc[0][0], sc[0][1]);
+#pragma unroll
+    for (int e = 2; e < 32; e += 2) cm = max3_f32(cm, sc[e >> 4][e & 15], sc[e >> 4][(e & 15) + 1]);
+    cm *= sl2e;
+    // the reference max moves only when some column outgrows it by 8 (p <= 2^8)
+    if (__any(cm > m + 8.f)) {
+      const float m_new = fmaxf(m, max_xor32(cm));
+      const float alpha = fast_exp2(m - (m_new == -INFINITY ? 0.f : m_new));   // 0 while m = -inf
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[b] *= alpha;
+    }
+    const float neg_m = m == -INFINITY ? 0.f : -m;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      // k index 8 half + j <-> position 16 w + 4 half + j (j < 4) or 8 further
+      float p[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) p[j] = fast_exp2(fmaf(sc[w >> 1][8 * (w & 1) + j], sl2e, neg_m));
+      pb[w] = smath<Tag>::pack8(p);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) l = M::add2(pb[w][j], ones, l);   // of the rounded P that multiplies V
+    }
+  };
+  // O^T += V^T.P of the chunk in a slot
+  auto values = [&](int slot) {
+    const char* const base = lds + slot * S::SLOT;
+    uint2 vf[2][NB][2];
+    auto read = [&](int w) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const char* const vp = base + va[b] + 16 * w * RB;
+        vf[w & 1][b][0] = lds_read_tr16(vp);
+        vf[w & 1][b][1] = lds_read_tr16(vp + 8 * RB);
+      }
+    };
+    read(0);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      if (w + 1 < 4) read(w + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const uint2 lo = vf[w & 1][b][0], hi = vf[w & 1][b][1];
+        acc[b] = M::mfma(su32x4_t{lo.x, lo.y, hi.x, hi.y}, pb[w], acc[b]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // Chunk k of the range (relative to c_begin) lies in ring slot k % RING.
+  const int n = c_end - c_begin;
+  const int n_wave = wave_busy ? min(c_end - 1, wave_last / CK) - c_begin + 1 : 0;   // this wave's chunks
+  for (int k = 0; k < n; ++k) {
+    // the wave's loads of chunk k have landed and its LDS reads of chunk k - 1 are done:
+    // behind the barrier all of chunk k is in LDS and the slot of chunk k - 1 is free
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (k + 1 < n) issue(c_begin + k + 1, (k + 1) % S::RING);
+    if (k < n_wave) {
+      const int slot = k % S::RING;
+      scores(slot);
+      softmax(c_begin + k);
+      values(slot);
+    }
+  }
+
+  l = sum_xor32(l);
+  if (!mine) return;
+  const int row = row0 + my_row;
+  const int pbeg = a.row_part_off[row], nparts = a.row_part_off[row + 1] - pbeg;
+  if (nparts == 1) {                            // the whole row: final output
+    const float inv = 1.f / l;
+    char* const orow = a.out + (int64_t)row * a.out_row_bytes + (int64_t)hd * RB + 8 * half;
+    typedef scalar_t s4_t __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        s4_t o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = (scalar_t)(acc[b][4 * g + j] * inv);
+        st8_through(orow + 64 * b + 16 * g, o);
+      }
+  } else if (part < nparts) {                   // partial of a split row (rows ending before the part own no slot)
+    const int64_t slot_i = (int64_t)(pbeg + part) * a.num_heads + hd;
+    float* const dst = a.ws_acc + slot_i * D + 4 * half;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4_t*>(dst + 32 * b + 8 * g) =
+            float4_t{acc[b][4 * g], acc[b][4 * g + 1], acc[b][4 * g + 2], acc[b][4 * g + 3]};
+    if (half == 0) *reinterpret_cast<float2*>(a.ws_ml + slot_i * 2) = make_float2(m, l);
+  }
+}
+
+}  // namespace tb
+
+// ---------------------------------------------------------------------------
+// Host side: the work list (no device call) and the launch.
+
+namespace {
+
+constexpr int COLS = tb::cshape<64>::COLS, CHUNK = tb::cshape<64>::CK;
+static_assert(COLS == tb::cshape<128>::COLS && CHUNK == tb::cshape<128>::CK, "one work list for both head dims");
+
+struct col_entry {
+  int seq, kvh, col0, part, chunks;
+};
+
+bool columns_args_ok(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs, int32_t num_heads,
+                     int32_t num_kv_heads) {
+  if (num_seqs < 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads) return false;
+  if (num_seqs > 0 && (!pos0 || !new_rows)) return false;
+  for (int i = 0; i < num_seqs; ++i)
+    if (pos0[i] < 0 || new_rows[i] <= 0 || (int64_t)pos0[i] + new_rows[i] > (1 << 24) ||
+        (int64_t)new_rows[i] * (num_heads / num_kv_heads) > (1 << 28))
+      return false;
+  return true;
+}
+
+// The positions the last row of the columns from col0 on sees.
+int columns_limit(int pos0, int new_rows, int rep, int col0) {
+  return pos0 + std::min(col0 + COLS - 1, new_rows * rep - 1) / rep + 1;
+}
+
+}  // namespace
+
+extern "C" int32_t tb_prefill_columns_partition(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs,
+                                                int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                                                int32_t num_cus) {
+  if (!columns_args_ok(pos0, new_rows, num_seqs, num_heads, num_kv_heads) || num_cus <= 0) return TB_ERR_INVALID_ARG;
+  if (head_dim != 64 && head_dim != 128) return TB_ERR_INVALID_ARG;
+  const int rep = num_heads / num_kv_heads;
+  int64_t total = 0;
+  int longest = 0;
+  for (int i = 0; i < num_seqs; ++i)
+    for (int c = 0; c < new_rows[i] * rep; c += COLS) {
+      const int n = (columns_limit(pos0[i], new_rows[i], rep, c) + CHUNK - 1) / CHUNK;
+      total += (int64_t)n * num_kv_heads;
+      longest = std::max(longest, n);
+    }
+  const int whole = (longest + 1) * CHUNK;             // no row is split
+  const int64_t share = (total + num_cus - 1) / num_cus;   // chunks per CU
+  if (longest <= share) return whole;
+  // the scratch a split needs (partials of every row that is longer than a partition)
+  auto scratch = [&](int64_t part) {
+    int64_t parts = 0;
+    for (int i = 0; i < num_seqs; ++i)
+      for (int r = 0; r < new_rows[i]; ++r) parts += (pos0[i] + r + part) / part;
+    return parts * num_heads * (head_dim + 2) * 4;
+  };
+  int part = std::max(8, (int)((share + 1) / 2));
+  part = std::min(part, 16);
+  if (part < 16 && scratch((int64_t)part * CHUNK) > TB_NOALLOC_SCRATCH_BYTES) part = 16;
+  return part * CHUNK < whole ? part * CHUNK : whole;
+}
+
+extern "C" int32_t tb_build_prefill_columns_work(const int32_t* first_row, const int32_t* seq_index, const int32_t* pos0,
+                                                 const int32_t* new_rows, int32_t num_seqs, int32_t num_heads,
+                                                 int32_t num_kv_heads, int32_t partition_tokens, int32_t num_xcds,
+                                                 int32_t num_cus, int32_t* work, int32_t capacity, int32_t* count) {
+  if (!columns_args_ok(pos0, new_rows, num_seqs, num_heads, num_kv_heads) || !count || num_xcds <= 0 || num_cus <= 0)
+    return TB_ERR_INVALID_ARG;
+  if (num_seqs > 0 && (!first_row || !seq_index)) return TB_ERR_INVALID_ARG;
+  if (partition_tokens < CHUNK || partition_tokens % CHUNK) return TB_ERR_INVALID_ARG;
+  for (int i = 0; i < num_seqs; ++i)
+    if (first_row[i] < 0 || seq_index[i] < 0) return TB_ERR_INVALID_ARG;
+  const int rep = num_heads / num_kv_heads, pc = partition_tokens / CHUNK;
+  std::vector<col_entry> entries;
+  int64_t total = 0;
+  for (int h = 0; h < num_kv_heads; ++h)
+    for (int i = 0; i < num_seqs; ++i)
+      for (int c = 0; c < new_rows[i] * rep; c += COLS) {
+        const int n = (columns_limit(pos0[i], new_rows[i], rep, c) + CHUNK - 1) / CHUNK;
+        for (int p = 0; p * pc < n; ++p) {
+          entries.push_back({i, h, c, p, std::min(pc, n - p * pc)});
+          total += entries.back().chunks + 2;            // + 2: a workgroup's start and end
+        }
+      }
+  // Entry g runs on XCD g % num_xcds: the entries in (kv head, sequence) order are cut into
+  // runs of equal work, one per XCD, so that few K/V ranges pass through each L2.
+  const int X = num_xcds, per = std::max(1, num_cus / X);
+  std::vector<std::vector<col_entry>> bins(X);
+  int64_t at = 0;
+  for (const col_entry& e : entries) {
+    const int64_t w = e.chunks + 2;
+    bins[std::min<int64_t>(X - 1, (2 * at + w) * X / (2 * total))].push_back(e);
+    at += w;
+  }
+  size_t rounds = 0;
+  for (auto& b : bins) {
+    // longest first, and every second round of one entry per CU reversed: a CU holds two or
+    // three workgroups at once, and its long first one then has a short second one
+    std::stable_sort(b.begin(), b.end(), [](const col_entry& x, const col_entry& y) { return x.chunks > y.chunks; });
+    for (size_t r = per; r + per <= b.size(); r += 2 * per) std::reverse(b.begin() + r, b.begin() + r + per);
+    rounds = std::max(rounds, b.size());
+  }
+  const int64_t n = (int64_t)rounds * X;
+  if (n > INT32_MAX) return TB_ERR_INVALID_ARG;
+  *count = (int32_t)n;
+  if (!work) return TB_OK;                             // the count alone
+  if (n > capacity) return TB_ERR_INVALID_ARG;
+  for (size_t r = 0; r < rounds; ++r)
+    for (int x = 0; x < X; ++x) {
+      int32_t* w = work + 8 * (r * X + x);
+      if (r >= bins[x].size()) {
+        std::fill(w, w + 8, 0);                          // no rows: the workgroup ends at once
+        continue;
+      }
+      const col_entry& e = bins[x][r];
+      w[0] = first_row[e.seq];
+      w[1] = seq_index[e.seq];
+      w[2] = pos0[e.seq];
+      w[3] = new_rows[e.seq];
+      w[4] = e.col0;
+      w[5] = e.kvh;
+      w[6] = e.part;
+      w[7] = pc;
+    }
+  return TB_OK;
+}
+
+extern "C" int32_t tb_paged_prefill_columns(const void* q, int64_t q_row_stride, const void* pool, int64_t num_blocks,
+                                            void* out, int64_t out_row_stride, const int32_t* block_tables,
+                                            int32_t max_blocks_per_seq, const int32_t* work, int32_t num_work,
+                                            const int32_t* row_part_offsets, int32_t num_rows,
+                                            const int32_t* split_rows, int32_t num_split_rows,
+                                            int32_t max_parts_per_row, int32_t total_partitions, int32_t num_heads,
+                                            int32_t num_kv_heads, int32_t head_dim, int32_t block_size, float scale,
+                                            int32_t dtype, void* workspace, size_t workspace_bytes,
+                                            const float* rope_cos, const float* rope_sin, int32_t rope_max_position,
+                                            hipStream_t stream) {
+  using namespace tb;
+  TB_CHECK_ARG(num_work >= 0 && num_rows >= 0 && num_split_rows >= 0 && num_split_rows <= num_rows);
+  TB_CHECK_ARG(num_heads > 0 && num_kv_heads > 0 && num_heads % num_kv_heads == 0);
+  if (num_work == 0) return TB_OK;
+  if (dtype != TB_DTYPE_F16 && dtype != TB_DTYPE_BF16) return TB_ERR_UNSUPPORTED;
+  if (head_dim != 64 && head_dim != 128) return TB_ERR_UNSUPPORTED;
+  if (block_size < 16 || (block_size & (block_size - 1))) return TB_ERR_UNSUPPORTED;
+  TB_CHECK_ARG(q && pool && out && block_tables && work && row_part_offsets && num_rows > 0);
+  TB_CHECK_ARG(num_blocks > 0 && max_blocks_per_seq > 0 && max_parts_per_row >= 0 && total_partitions >= 0);
+  TB_CHECK_ARG(q_row_stride >= (int64_t)num_heads * head_dim && out_row_stride >= (int64_t)num_heads * head_dim);
+  TB_CHECK_ARG((((uintptr_t)q | (uintptr_t)pool | (uintptr_t)out | (uintptr_t)work) & 15u) == 0);
+  TB_CHECK_ARG((q_row_stride * 2) % 16 == 0 && (out_row_stride * 2) % 16 == 0);
+  TB_CHECK_ARG(num_split_rows == 0 || (split_rows && max_parts_per_row > 1));
+  TB_CHECK_ARG(((uintptr_t)split_rows & 15u) == 0);
+  TB_CHECK_ARG(!rope_cos == !rope_sin && (!rope_cos || rope_max_position > 0));
+  TB_CHECK_ARG((((uintptr_t)rope_cos | (uintptr_t)rope_sin) & 15u) == 0);
+  void* ws = nullptr;
+  if (max_parts_per_row > 1) {
+    const size_t need = tb_paged_attention_workspace_bytes(total_partitions, num_heads, head_dim);
+    ws = workspace;
+    if (!ws) {                                           // the library's static scratch
+      if (need > (size_t)TB_NOALLOC_SCRATCH_BYTES) return TB_ERR_SCRATCH;
+      const int32_t st = noalloc_scratch(stream, &ws);
+      if (st != TB_OK) return st;
+    } else {
+      TB_CHECK_ARG(workspace_bytes >= need && ((uintptr_t)ws & 15u) == 0);
+    }
+  }
+  cols_args a{};
+  a.q = static_cast<const char*>(q);
+  a.q_row_bytes = q_row_stride * 2;
+  a.pool = static_cast<const char*>(pool);
+  a.num_blocks = num_blocks;
+  a.out = static_cast<char*>(out);
+  a.out_row_bytes = out_row_stride * 2;
+  a.block_tables = block_tables;
+  a.max_nb = max_blocks_per_seq;
+  a.work = reinterpret_cast<const int4*>(work);
+  a.row_part_off = row_part_offsets;
+  a.ws_acc = static_cast<float*>(ws);
+  a.ws_ml = ws ? a.ws_acc + (size_t)total_partitions * num_heads * head_dim : nullptr;
+  a.num_heads = num_heads;
+  a.num_kv_heads = num_kv_heads;
+  a.rep = num_heads / num_kv_heads;
+  while ((1 << a.log2_bs) < block_size) ++a.log2_bs;
+  a.scale_log2e = scale * 1.4426950408889634f;
+  a.rope = rope_tables{rope_cos, rope_sin, rope_max_position};
+  const dim3 grid(num_work), block(64 * cshape<64>::NW);
+  const bool d64 = head_dim == 64;
+  if (dtype == TB_DTYPE_F16) {
+    if (d64) hipLaunchKernelGGL((paged_prefill_columns_kernel<f16_t, 64>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((paged_prefill_columns_kernel<f16_t, 128>), grid, block, 0, stream, a);
+  } else {
+    if (d64) hipLaunchKernelGGL((paged_prefill_columns_kernel<bf16_t, 64>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((paged_prefill_columns_kernel<bf16_t, 128>), grid, block, 0, stream, a);
+  }
+  if (num_split_rows > 0)
+    combine_split_rows(dtype, head_dim, num_heads, out, out_row_stride * 2, split_rows, num_split_rows, a.ws_acc, a.ws_ml,
+                       stream);
+  TB_RETURN_LAUNCH_STATUS();
+}

@@ -94,11 +94,15 @@ class PagedKVCache:
             if r is not None and any(qlens) and all(
                     n == 0 or (n >= 16 and c <= r.max_context) for n, c in zip(qlens, context_lens)):
                 route = r
+        columns = None
+        if num_heads is not None and context_lens is not None and self.device.type == "cuda" and route is None:
+            columns = ops.columns_route(self.dtype, num_heads, self.n_kv_heads, self.head_dim, self.block_size,
+                                        self.device)
         meta = build_step_metadata(positions if host_positions is None else host_positions,
                                    seq_slices, block_tables, context_lens,
                                    block_size=self.block_size, num_blocks=self.num_blocks,
                                    partition_tokens=self.partition_tokens, rows_per_item=rows_per_item,
-                                   tile_prefill=tile, prefill_route=route)
+                                   tile_prefill=tile, prefill_route=route, columns_route=columns)
         if num_heads is not None and context_lens is not None and self.device.type == "cuda" and tile \
                 and route is None:
             # whole prefills beside a run of decode rows: tb_paged_prefill and the

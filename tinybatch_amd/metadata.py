@@ -105,6 +105,11 @@ class StepMetadata:
     num_prefill_work: int = 0
     prefill_max_tiles: int = 0
     prefill_work: torch.Tensor | None = None
+    # prefill sequences of any context served by tb_paged_prefill_columns
+    # (build_step_metadata's columns_route): its work list [n, 8] and partition length
+    columns_work_np: np.ndarray | None = None
+    num_columns_work: int = 0
+    columns_work: torch.Tensor | None = None
     # a mixed step served as sub-steps (split_step_parts): (first row, end row, the
     # sub-step's metadata with rows counted from the first row); the arrays above
     # still describe the whole step (its slot mapping serves the append)
@@ -117,8 +122,8 @@ class StepMetadata:
             m.to(device)
         parts = [self.slot_mapping_np, self.block_tables_np.reshape(-1), self.work_np.reshape(-1),
                  self.row_part_off_np, self.prefill_tiles_np.reshape(-1), self.split_rows_np.reshape(-1)]
-        extra = [x for x in (self.decode_plan_np, self.slot_map_np, self.prefill_work_np, self.decode_counts_np,
-                             self.decode_segments_np) if x is not None]
+        extra = [x for x in (self.decode_plan_np, self.slot_map_np, self.prefill_work_np, self.columns_work_np,
+                             self.decode_counts_np, self.decode_segments_np) if x is not None]
         parts += extra
         sizes = [pad4(p.size) for p in parts]
         host = np.zeros(sum(sizes), dtype=np.int32)
@@ -145,6 +150,9 @@ class StepMetadata:
             k += 1
         if self.prefill_work_np is not None:
             self.prefill_work = buf.narrow(0, int(offs[k]), parts[k].size)
+            k += 1
+        if self.columns_work_np is not None:
+            self.columns_work = buf.narrow(0, int(offs[k]), parts[k].size)
             k += 1
         if self.decode_segments_np is not None:
             counts = buf.narrow(0, int(offs[k]), parts[k].size)
@@ -211,6 +219,52 @@ class PrefillRoute(NamedTuple):
     num_xcds: int = 1
 
 
+class ColumnsRoute(NamedTuple):
+    """Where prefill sequences of any context go to tb_paged_prefill_columns in place of
+    tiles: the step's heads and head dim, the GPU's XCDs and CUs (ops.columns_route)."""
+    num_heads: int
+    num_kv_heads: int
+    head_dim: int
+    num_xcds: int
+    num_cus: int
+
+
+def _i32_columns(*columns):
+    """The columns as int32 arrays and their pointers."""
+    import ctypes
+
+    cols = [np.ascontiguousarray(np.asarray(x, dtype=np.int32).reshape(-1)) for x in columns]
+    return cols, [c.ctypes.data_as(ctypes.c_void_p) for c in cols]
+
+
+def columns_partition(pos0s, new_rows, route: ColumnsRoute) -> int:
+    """tb_prefill_columns_partition: positions per partition of the step's column rows."""
+    from . import _lib
+
+    cols, ptrs = _i32_columns(pos0s, new_rows)
+    p = int(_lib.lib().tb_prefill_columns_partition(*ptrs, cols[0].size, route.num_heads, route.num_kv_heads,
+                                                    route.head_dim, route.num_cus))
+    if p < 0:
+        _lib.check(p, "tb_prefill_columns_partition")
+    return p
+
+
+def build_columns_work(first_rows, seqs, pos0s, new_rows, partition: int, route: ColumnsRoute) -> np.ndarray:
+    """tb_build_prefill_columns_work: int32 [n, 8], entry g for XCD g % route.num_xcds."""
+    import ctypes
+
+    from . import _lib
+
+    cols, ptrs = _i32_columns(first_rows, seqs, pos0s, new_rows)
+    args = (*ptrs, cols[0].size, route.num_heads, route.num_kv_heads, partition, route.num_xcds, route.num_cus)
+    lib, n = _lib.lib(), ctypes.c_int32()
+    _lib.check(lib.tb_build_prefill_columns_work(*args, None, 0, ctypes.byref(n)), "tb_build_prefill_columns_work")
+    work = np.zeros((max(n.value, 1), 8), dtype=np.int32)
+    _lib.check(lib.tb_build_prefill_columns_work(*args, work.ctypes.data_as(ctypes.c_void_p), n.value, ctypes.byref(n)),
+               "tb_build_prefill_columns_work")
+    return work[:n.value]
+
+
 def build_prefill_work(first_rows, seqs, pos0s, new_rows, *, num_kv_heads: int, head_dim: int,
                        num_xcds: int = 1) -> tuple[np.ndarray, int]:
     """tb_build_prefill_work: one entry (first row, sequence, pos0, new rows | pair <<
@@ -256,8 +310,12 @@ def _host_positions(positions) -> np.ndarray:
 def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, block_size: int,
                         num_blocks: int, partition_tokens: int, num_tokens: int | None = None,
                         validate_attention: bool = True, rows_per_item: int = 1,
-                        tile_prefill: bool = False, prefill_route: PrefillRoute | None = None) -> StepMetadata:
+                        tile_prefill: bool = False, prefill_route: PrefillRoute | None = None,
+                        columns_route: ColumnsRoute | None = None) -> StepMetadata:
     """Build the per-step arrays (host side). See the module docstring. With
+    ``columns_route``, sequences of >= 16 new rows go to tb_paged_prefill_columns
+    (columns_work_np) in place of tiles and work items; their rows count partitions of its
+    partition length. With
     ``prefill_route``, sequences of >= 16 new rows whose context is at most its
     max_context go to tb_paged_prefill whole (prefill_work_np); their rows get no
     work items, tiles or partition slots."""
@@ -324,6 +382,8 @@ def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, bl
     row_ctx_by_row = np.zeros(T, dtype=np.int64)
     tiles: list[tuple[int, int, int, int, int]] = []
     stream_seqs: list[tuple[int, int, int, int]] = []
+    column_seqs: list[tuple[int, int, int, int]] = []
+    columns_work = None
     tiled = np.zeros(T, dtype=bool)
     nparts_by_row = np.zeros(T, dtype=np.int64)
     if tot and context_lens is not None:
@@ -349,6 +409,17 @@ def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, bl
                     tiled[s0:s0 + n] = True               # served by tb_paged_prefill
                     nparts_by_row[s0:s0 + n] = 0
                     stream_seqs.append((s0, b, c - n, n))
+        if columns_route is not None:
+            for b in range(B):
+                n, c = int(qlens[b]), int(ctx[b])
+                if n >= 16 and not tiled[int(starts[b])]:
+                    column_seqs.append((int(starts[b]), b, c - n, n))
+            if column_seqs:
+                part = columns_partition([x[2] for x in column_seqs], [x[3] for x in column_seqs], columns_route)
+                for s0, _, _, n in column_seqs:
+                    tiled[s0:s0 + n] = True               # served by tb_paged_prefill_columns
+                    nparts_by_row[s0:s0 + n] = (row_ctx_by_row[s0:s0 + n] + part - 1) // part
+                columns_work = build_columns_work(*zip(*column_seqs), part, columns_route)
         if tile_prefill:
             for b in range(B):
                 n, c = int(qlens[b]), int(ctx[b])
@@ -443,6 +514,8 @@ def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, bl
         prefill_work_np=prefill_work,
         num_prefill_work=0 if prefill_work is None else int(prefill_work.shape[0]),
         prefill_max_tiles=prefill_tiles_max,
+        columns_work_np=columns_work,
+        num_columns_work=0 if columns_work is None else int(columns_work.shape[0]),
     )
 
 
@@ -760,7 +833,8 @@ def attach_xcd_slot_map(meta: StepMetadata, *, num_heads: int, num_kv_heads: int
     uploaded by ``meta.to``. Applies to 16-bit steps without prefill tiles, with at most
     16 query heads per kv head and no capacity counts; returns whether it does."""
     if (dtype not in (torch.float16, torch.bfloat16) or meta.num_prefill_tiles > 0 or meta.num_split_rows == 0
-            or num_heads // num_kv_heads > 16 or meta.device_buffer is not None or meta.num_work_items == 0):
+            or num_heads // num_kv_heads > 16 or meta.device_buffer is not None or meta.num_work_items == 0
+            or meta.num_columns_work > 0):
         return False
     if meta.max_parts_per_row > MERGED_MAX_PARTS:
         # the merged launch counts a row's partitions in 8-bit fields; the combine

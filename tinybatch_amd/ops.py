@@ -267,6 +267,24 @@ def prefill_route(dtype: torch.dtype, num_heads: int, num_kv_heads: int, head_di
     return PrefillRoute(num_kv_heads, head_dim, max_ctx, xcds)
 
 
+def columns_route(dtype: torch.dtype, num_heads: int, num_kv_heads: int, head_dim: int, block_size: int,
+                  device: torch.device):
+    """The ColumnsRoute (build_step_metadata's columns_route) that sends prefill sequences of
+    any context to tb_paged_prefill_columns for this geometry, or None where that kernel
+    does not serve it (fp32, other head dims, blocks of fewer than 16 positions).
+
+    Against the 64-row tiles it replaces (bf16, us per layer): four prompts of 1746..3738
+    tokens at 14 / 2 heads of 64: 90 against 135; three of 5300..7333 at 32 / 8 heads of
+    128: 1070 against 3550."""
+    from .metadata import ColumnsRoute
+
+    if (dtype not in (torch.float16, torch.bfloat16) or num_kv_heads <= 0 or num_heads % num_kv_heads
+            or head_dim not in (64, 128) or block_size < 16 or block_size & (block_size - 1)):
+        return None
+    d = decode_device(device)
+    return ColumnsRoute(num_heads, num_kv_heads, head_dim, d.num_xcds if d.merge_in_kernel else 1, d.workgroups)
+
+
 def decode_kernel_preferred(meta: StepMetadata, *, num_kv_heads: int, head_dim: int, dtype: torch.dtype,
                             min_bytes: int = DECODE_KERNEL_MIN_BYTES) -> bool:
     """Whether a step is served faster by the streaming decode kernel: a decode-only
@@ -537,7 +555,7 @@ def paged_attention(q: torch.Tensor, pool: torch.Tensor, meta: StepMetadata, *, 
             # whole prefill sequences only: tb_paged_prefill reads their new rows from
             # k_new / v_new (K rotated in the kernel with ``rope``) and stores them
             prefill_fused = True
-        elif not meta.decode_only or meta.num_prefill_tiles or meta.num_prefill_work:
+        elif not meta.decode_only or meta.num_prefill_tiles or meta.num_prefill_work or meta.num_columns_work:
             raise ValueError("fused append needs a decode-only step (one query row per sequence) or a step of "
                              "whole prefills only")
         sm = meta.slot_mapping_np
@@ -573,6 +591,24 @@ def paged_attention(q: torch.Tensor, pool: torch.Tensor, meta: StepMetadata, *, 
             meta.max_blocks_per_seq, meta.prefill_work.data_ptr(), meta.num_prefill_work, meta.prefill_max_tiles,
             num_heads, hkv, d, bs, float(scale), _lib.DTYPE_CODE[q.dtype],
             *((ksp, ks, vsp, vs) if prefill_fused else (None, 0, None, 0)), *tail[1:]), "tb_paged_prefill")
+    if meta.num_columns_work:   # prefill rows of any context; a step of nothing else merges its split rows here
+        if meta.columns_work is None:
+            raise ValueError("metadata has not been uploaded (call meta.to(device))")
+        if noalloc and workspace is not None:
+            raise ValueError("noalloc takes no workspace")
+        if workspace is None and not noalloc:
+            workspace = workspace_for(meta, num_heads, d, q.device)
+        last = not meta.num_work_items and not meta.num_prefill_tiles
+        _lib.check(_lib.lib().tb_paged_prefill_columns(
+            q.data_ptr(), qs, pool.data_ptr(), nb, out.data_ptr(), os_, meta.block_tables.data_ptr(),
+            meta.max_blocks_per_seq, meta.columns_work.data_ptr(), meta.num_columns_work, meta.row_part_off.data_ptr(), T,
+            meta.split_rows.data_ptr(), meta.num_split_rows if last else 0, meta.max_parts_per_row,
+            meta.total_partitions, num_heads, hkv, d, bs, float(scale), _lib.DTYPE_CODE[q.dtype],
+            None if workspace is None else workspace.data_ptr(),
+            0 if workspace is None else workspace.numel() * workspace.element_size(), *tail[1:]),
+            "tb_paged_prefill_columns")
+        if last:
+            return out
     if noalloc:
         if workspace is not None:
             raise ValueError("noalloc takes no workspace")
