@@ -60,10 +60,13 @@ __device__ __forceinline__ void st16(void* p, const vec16& r) {
 // - the 1024-block copy over 24 pools: 73.0 against 86.9 us;
 // - the prefill rows of 8 x 512 bf16: 11.9 against 12.5 us per layer.
 // The 16-byte form is one vector store instruction; the compiler does not count
-// it in its own waits, so any later wait it makes only waits longer.
+// it in its own waits, so any later wait it makes only waits longer. Nor does it see
+// that the store still reads its data registers for two wait states (stores of more than
+// 8 bytes): a vector instruction right behind it that wrote the last of them was seen
+// to change the fourth word stored. The s_nop 1 is those two wait states.
 __device__ __forceinline__ void st16_through(void* p, const vec16& r) {
   const u32x4_t v = {r.w[0], r.w[1], r.w[2], r.w[3]};
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
 }
 template <typename T>
 __device__ __forceinline__ void st8_through(void* p, const T& r) {
@@ -79,7 +82,7 @@ __device__ __forceinline__ void st_through(void* p, const T& r) {
     st8_through(p, r);
   } else {
     const u32x4_t v = __builtin_bit_cast(u32x4_t, r);
-    asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
   }
 }
 
