@@ -250,8 +250,8 @@ int32_t tb_paged_prefill(const void* q, int64_t q_row_stride, void* pool, int64_
                          const float* rope_cos, const float* rope_sin, int32_t rope_max_position,
                          hipStream_t stream);
 /* K2 for prefill rows of any context (reference src/tinybatch/model.py:130-147), column
- * tiles: fp16 / bf16, head_dim 64 or 128, block_size a power of two >= 16, any number of
- * query heads per kv head (TB_ERR_UNSUPPORTED otherwise: use tb_paged_attention's tiles).
+ * tiles: head_dim 64 or 128, block_size a power of two >= 16, any number of query heads
+ * per kv head (TB_ERR_UNSUPPORTED otherwise: use tb_paged_attention).
  * The rows it serves must not also be given to tb_paged_attention as work items or tiles.
  * The K/V of the step's new rows must already be in the pool (append first).
  *   work: tb_build_prefill_columns_work's list (device memory, 16-byte aligned), num_work

@@ -28,8 +28,8 @@
 // Prefill tiles (fp16 / bf16): paged_prefill_mfma_kernel, a flash-style
 // workgroup per (64 query rows of one sequence, query head) that walks the
 // causal range in 64-position chunks staged in LDS (see the kernel).
-// fp32: paged_attn_valu_kernel, fp32 FMAs on the VALU (no fp32 MFMA of the
-// needed precision on CDNA4), same decomposition.
+// fp32: paged_attn_f32_kernel, the fp32 MFMA (fp32 products and sums), same
+// decomposition with one query row per item.
 // Positions >= the row's context are never loaded from the pool (stale slots
 // may hold any bits, NaN included): their scores are -inf, so p = 0, and what
 // stands in for their V rows is finite.
@@ -104,208 +104,203 @@ struct attn_args {
 
 
 // ---------------------------------------------------------------------------
-// fp32 path: single pass, online softmax per chunk, fp32 FMAs.
-template <typename Tag, int D>
-struct valu_shape {
-  static constexpr int EB = elem<Tag>::bytes;
-  static constexpr int EPL = 16 / EB;     // elements per lane per load
-  static constexpr int LPT = D / EPL;     // lanes per token row
-  static constexpr int TPL = 64 / LPT;    // tokens per wave load
-  static constexpr int CH_LOADS = 8;      // wave loads of K (and of V) per chunk
-  static constexpr int CH = CH_LOADS * TPL;  // tokens per chunk
-  static_assert(LPT >= 1 && LPT <= 64 && (64 % LPT) == 0, "lane split");
+// fp32 path. A workgroup of NW waves owns one work item (one query row, kv head, group of
+// heads, partition); wave w takes positions 16 w .. 16 w + 15 of every 16 NW. Both contractions run on
+// v_mfma_f32_16x16x4_f32 (fp32 products and sums), the heads as the 16 columns:
+//   S^T[pos][head]  = K[pos][:] . q[head][:]    A: lane (lg, lc) K[pos lc][16 c + 4 lg + i]
+//   O^T[d][head]   += V^T[d][pos] . P^T[pos][head]  A: V[pos 4 lg + j][4 lc + i], B: the S^T registers
+// (k index lg of a product stands for dim 16 c + 4 lg + i, or position 4 lg + j, in both
+// operands, so every operand is a whole 16-byte load used component by component). A
+// score's dims are summed in chains of 8. The waves' states merge in LDS.
+//
+// Bound by latency: at 8 rows of up to 250 positions a call is one chain of table read, K/V
+// read, 32 products a wave and the merge on 16 CUs. us per layer in a
+// graph: 8.4 (one wave per item walking its partition 32 positions at a time, dot products
+// reduced across lanes: 32.5).
+template <int D, int NW_>
+struct f32_shape {
+  static constexpr int RB = 4 * D;         // bytes per row
+  static constexpr int KC = D / 16;        // 16-byte K chunks of a lane (dims 16 c + 4 lg ..)
+  static constexpr int VC = D / 64;        // 16-byte V chunks of a lane per row (dims 64 c + 4 lc ..)
+  static constexpr int NW = NW_;           // waves per workgroup
+  static constexpr int SPAN = 16 * NW;     // positions in flight
+  static constexpr int PITCH = D + 4;      // floats per (wave, head) row of the merge
 };
 
-// End of a VALU work item. acc[h][e] holds, in lanes 0..LPT-1 (column j = lane),
-// the unnormalised output of head h over the partition for dims j*EPL..;
-// m[h] / l[h] (wave-uniform) are its max (base-2 domain) and sum. One
-// partition: write the output. Several: write the partial for the combine.
-template <typename Tag, int D, int REP, int EPL, int LPT>
-__device__ __forceinline__ void finish_valu(const attn_args& a, int row, int part, int head0, int lane,
-                                            float (&acc)[REP][EPL], const float (&m)[REP],
-                                            const float (&l)[REP]) {
-  const int j = lane % LPT;
-  if (lane >= LPT) return;
-  const int pbeg = a.row_part_off[row];
-  const int nparts = a.row_part_off[row + 1] - pbeg;
-  if (nparts == 1) {
-    char* orow = a.out + row * a.out_row_bytes + j * 16;
-#pragma unroll
-    for (int h = 0; h < REP; ++h) {
-      const float inv = 1.f / l[h];
-      vec16 o;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o.w[e] = __float_as_uint(acc[h][e] * inv);
-      st16_through(orow + (int64_t)(head0 + h) * D * 4, o);
-    }
-    return;
-  }
-  const int64_t pidx = pbeg + part;
-#pragma unroll
-  for (int h = 0; h < REP; ++h) {
-    float* dst = a.ws_acc + (pidx * a.num_heads + head0 + h) * D + j * EPL;
-#pragma unroll
-    for (int e = 0; e < EPL; e += 4)
-      *reinterpret_cast<float4*>(dst + e) = make_float4(acc[h][e], acc[h][e + 1], acc[h][e + 2], acc[h][e + 3]);
-  }
-  if (lane == 0) {
-#pragma unroll
-    for (int h = 0; h < REP; ++h)
-      *reinterpret_cast<float2*>(a.ws_ml + (pidx * a.num_heads + head0 + h) * 2) = make_float2(m[h], l[h]);
-  }
-}
+template <int D, int NW_>
+__global__ __launch_bounds__(64 * NW_) void paged_attn_f32_kernel(const attn_args a) {
+  using S = f32_shape<D, NW_>;
+  constexpr int RB = S::RB, KC = S::KC, VC = S::VC, NW = S::NW;
+  extern __shared__ __align__(16) float f32_lds[];   // [wave][group][PITCH], then [wave][16] (max, sum)
 
-template <typename Tag, int D, int REP>
-__global__ __launch_bounds__(64) void paged_attn_valu_kernel(const attn_args a) {
-  using S = valu_shape<Tag, D>;
-  constexpr int EB = S::EB, EPL = S::EPL, LPT = S::LPT, TPL = S::TPL;
-  constexpr int CH_LOADS = S::CH_LOADS, CH = S::CH;
-  static_assert(EB == 4, "the 16-bit types use paged_attn_mfma_kernel");
-
-  const int lane = threadIdx.x;
-  const int j = lane % LPT;  // 16-byte column of the token row
-  const int g = lane / LPT;  // token slot inside one wave load
-
-  const int4 wi = a.work[blockIdx.x];   // one row per item on this path; the array holds the grid's capacity
-  if (a.counts && (int)blockIdx.x >= a.counts[0]) return;   // beyond this step's work items
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, lc = lane & 15, lg = lane >> 4;
+  const int4 wi = a.work[blockIdx.x];      // one row per item on this path; the array holds the grid's capacity
+  if (a.counts && (int)blockIdx.x >= a.counts[0]) return;   // beyond this step's work items (whole workgroup)
   const int row = wi.x, seq = wi.y, part = wi.z & 0xFFFFFF, ctx = wi.w;
-  const int kvh = blockIdx.y;
-  const int head0 = kvh * a.rep + blockIdx.z * REP;
-
+  const int kvh = blockIdx.y, R = a.group;
+  const int head0 = kvh * a.rep + blockIdx.z * R;
   const int p0 = part * a.part_tokens;
   const int p1 = min(p0 + a.part_tokens, ctx);
   const int bs = 1 << a.log2_bs;
+  const int pbeg = a.row_part_off[row], nparts = a.row_part_off[row + 1] - pbeg;
 
-  // Block-table entries of this partition: lane l holds entry p0/BS + l.
-  const int blk_first = p0 >> a.log2_bs;
-  const int blk_count = ((p1 - 1) >> a.log2_bs) - blk_first + 1;  // <= 64 (host-checked)
-  int my_blk = 0;
-  if (lane < blk_count) {
-    my_blk = a.block_tables[(int64_t)seq * a.max_nb + blk_first + lane];
-    if (my_blk < 0 || my_blk >= a.num_blocks) my_blk = 0;  // host validates; stay inside the pool
-  }
-
-  const int64_t tile_bytes = (int64_t)bs * D * EB;
+  const int64_t tile_bytes = (int64_t)bs * RB;
   const int64_t blk_bytes = 2 * (int64_t)a.num_kv_heads * tile_bytes;
   const int64_t v_off = (int64_t)a.num_kv_heads * tile_bytes;
-  const char* pool_kvh = a.pool + kvh * tile_bytes + j * 16;
-  const int new_pos = ctx - 1;
-  const bool fused = (a.k_new != nullptr);
-  const char* k_new_row = fused ? a.k_new + row * a.k_new_row_bytes + (int64_t)kvh * D * EB + j * 16 : nullptr;
-  const char* v_new_row = fused ? a.v_new + row * a.v_new_row_bytes + (int64_t)kvh * D * EB + j * 16 : nullptr;
+  char* const pool_kvh = a.pool + kvh * tile_bytes;
+  const int32_t* const table = a.block_tables + (int64_t)seq * a.max_nb;
+  const int new_pos = a.k_new ? ctx - 1 : -1;          // the fused append's position
+  const char* const k_new_row = a.k_new + row * a.k_new_row_bytes + (int64_t)kvh * RB;
+  const char* const v_new_row = a.v_new + row * a.v_new_row_bytes + (int64_t)kvh * RB;
+  auto slot_of = [&](int pos) {            // the position's row in the pool (K)
+    int b = table[pos >> a.log2_bs];
+    b = (b < 0 || b >= a.num_blocks) ? 0 : b;          // host validates; stay inside the pool
+    return pool_kvh + b * blk_bytes + (int64_t)(pos & (bs - 1)) * RB;
+  };
 
-  vec16 qv[REP];
-  {
-    const char* qrow = a.q + row * a.q_row_bytes + j * 16;
+  // q (B operand: lane holds head lc's dims 16 c + 4 lg ..)
+  vec16 q[KC];
 #pragma unroll
-    for (int h = 0; h < REP; ++h) qv[h] = ld16(qrow + (int64_t)(head0 + h) * D * EB);
+  for (int c = 0; c < KC; ++c) q[c] = zero16();
+  if (lc < R) {
+    const char* qrow = a.q + row * a.q_row_bytes + (int64_t)(head0 + lc) * RB + 16 * lg;
+#pragma unroll
+    for (int c = 0; c < KC; ++c) q[c] = ld16(qrow + 64 * c);
   }
-  // RoPE: chunk j of the first half pairs with chunk j + LPT/2 of the second,
-  // held by lane ^ LPT/2 of the same token slot (every lane holds its chunk)
-  vec16 k_new_rot = zero16();
-  if (a.rope.cos) {
-    const bool first = j < LPT / 2;
-    const int64_t r = a.rope.row(ctx - 1, D / 2) + (first ? j : j - LPT / 2) * 4;
-    auto rotate = [&](vec16& x) {
-      vec16 y;
+
+  float m = -INFINITY, l = 0.f;            // of head lc; l: this lane's share
+  float4_t acc[4 * VC];                    // O^T: dims 64 c + 4 (4 lg + j) + i of head lc, at [4 c + i][j]
 #pragma unroll
-      for (int e = 0; e < 4; ++e) y.w[e] = (uint32_t)__shfl_xor((int)x.w[e], LPT / 2);
-      if (first) rope_pair<float>(x, y, a.rope.cos + r, a.rope.sin + r);
-      else rope_pair<float>(y, x, a.rope.cos + r, a.rope.sin + r);
-    };
+  for (int e = 0; e < 4 * VC; ++e) acc[e] = float4_t{0.f, 0.f, 0.f, 0.f};
+  bool rotated = false;
+  for (int t0 = p0 + 16 * wave; t0 < p1; t0 += S::SPAN) {   // wave-uniform
+    const int kpos = min(t0 + lc, p1 - 1), vpos = t0 + 4 * lg;   // V: positions vpos .. vpos + 3, one block
+    char* const kslot = slot_of(kpos);
+    char* const vslot = slot_of(min(vpos, p1 - 1) & ~3) + v_off;
+    const char* const ksrc = (kpos == new_pos ? k_new_row : kslot) + 16 * lg;
+    vec16 k[KC], v[4][VC];
 #pragma unroll
-    for (int h = 0; h < REP; ++h) rotate(qv[h]);
-    if (fused) {
-      k_new_rot = ld16(k_new_row);
-      rotate(k_new_rot);
+    for (int c = 0; c < KC; ++c) k[c] = ld16(ksrc + 64 * c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const char* const src = (vpos + j == new_pos ? v_new_row : vslot + (vpos + j < p1 ? j * RB : 0)) + 16 * lc;
+#pragma unroll
+      for (int c = 0; c < VC; ++c) v[j][c] = ld16(src + 256 * c);
     }
-  }
-
-  float m_run[REP], l_run[REP], acc[REP][EPL];
+    if (a.rope.cos) {                      // chunk c pairs with chunk c + KC/2 (dims i and i + D/2) in the same lane
+      if (!rotated && lc < R) {
+        const int64_t r = a.rope.row(ctx - 1, D / 2) + 4 * lg;
 #pragma unroll
-  for (int h = 0; h < REP; ++h) {
-    m_run[h] = -INFINITY;
-    l_run[h] = 0.f;
+        for (int c = 0; c < KC / 2; ++c)
+          rope_pair<float>(q[c], q[c + KC / 2], a.rope.cos + r + 16 * c, a.rope.sin + r + 16 * c);
+      }
+      rotated = true;
+      if (kpos == new_pos) {
+        const int64_t r = a.rope.row(ctx - 1, D / 2) + 4 * lg;
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) acc[h][e] = 0.f;
-  }
-
-  int64_t new_off = 0;
-  if (fused) {
-    const int nb = __shfl(my_blk, ((new_pos - p0) >> a.log2_bs) & 63);
-    new_off = (int64_t)nb * blk_bytes + (int64_t)(new_pos & (bs - 1)) * (D * EB);
-  }
-
-  for (int c0 = p0; c0 < p1; c0 += CH) {
-    vec16 kbuf[CH_LOADS], vbuf[CH_LOADS];
-#pragma unroll
-    for (int i = 0; i < CH_LOADS; ++i) {
-      const int tau = c0 + i * TPL + g;
-      const int blk = __shfl(my_blk, ((tau - p0) >> a.log2_bs) & 63);
-      const int64_t off = (int64_t)blk * blk_bytes + (int64_t)(tau & (bs - 1)) * (D * EB);
-      const char* kp = pool_kvh + off;
-      const char* vp = kp + v_off;
-      if (fused && tau == new_pos) { kp = k_new_row; vp = v_new_row; }
-      if (tau < p1) { kbuf[i] = ld16(kp); vbuf[i] = ld16(vp); }
-      else { kbuf[i] = zero16(); vbuf[i] = zero16(); }
-      if (fused && a.rope.cos && tau == new_pos) kbuf[i] = k_new_rot;
+        for (int c = 0; c < KC / 2; ++c)
+          rope_pair<float>(k[c], k[c + KC / 2], a.rope.cos + r + 16 * c, a.rope.sin + r + 16 * c);
+      }
     }
-    if (fused) {
+    if (new_pos >= t0 && new_pos < t0 + 16 && blockIdx.z == 0) {   // the fused append: lanes holding the new row store it
+      if (t0 + lc == new_pos) {
 #pragma unroll
-      for (int i = 0; i < CH_LOADS; ++i) {
-        if (c0 + i * TPL + g == new_pos) {
-          char* kp = const_cast<char*>(pool_kvh) + new_off;
-          st16_through(kp, kbuf[i]);
-          st16_through(kp + v_off, vbuf[i]);
+        for (int c = 0; c < KC; ++c) st16_through(kslot + 16 * lg + 64 * c, k[c]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (vpos + j == new_pos) {
+#pragma unroll
+          for (int c = 0; c < VC; ++c) st16_through(vslot + j * RB + 16 * lc + 256 * c, v[j][c]);
         }
-      }
     }
-    float s[CH_LOADS][REP];
+    float4_t sh[2];                        // chains of 8 dims, added pairwise
 #pragma unroll
-    for (int i = 0; i < CH_LOADS; ++i) {
-      const bool valid = (c0 + i * TPL + g) < p1;
+    for (int h = 0; h < 2; ++h) {
+      float4_t sc[KC];
 #pragma unroll
-      for (int h = 0; h < REP; ++h) {
-        float d = 0.f;
+      for (int c = 0; c < KC; ++c) {
+        sc[c] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) d = fmaf(bits_to_f32(qv[h].w[e]), bits_to_f32(kbuf[i].w[e]), d);
-        d = group_sum<LPT>(d);
-        s[i][h] = valid ? d * a.scale_log2e : -INFINITY;
+        for (int i = 2 * h; i < 2 * h + 2; ++i)
+          sc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(bits_to_f32(k[c].w[i]), bits_to_f32(q[c].w[i]), sc[c], 0, 0, 0);
       }
+#pragma unroll
+      for (int st = 1; st < KC; st *= 2)
+#pragma unroll
+        for (int c = 0; c < KC; c += 2 * st) sc[c] += sc[c + st];
+      sh[h] = sc[0];
     }
+    float4_t s = sh[0] + sh[1];            // positions t0 + 4 lg + j of head lc
 #pragma unroll
-    for (int h = 0; h < REP; ++h) {
-      float cm = s[0][h];
+    for (int j = 0; j < 4; ++j) s[j] = vpos + j < p1 ? s[j] * a.scale_log2e : -INFINITY;
+    const float cm = max_xor32(max_xor16(max_f32(max_f32(s[0], s[1]), max_f32(s[2], s[3]))));
+    const float m_new = max_f32(m, cm);    // finite: the tile's first position is visible
+    const float alpha = fast_exp2(m - m_new);
+    m = m_new;
+    l *= alpha;
 #pragma unroll
-      for (int i = 1; i < CH_LOADS; ++i) cm = fmaxf(cm, s[i][h]);
-      cm = cross_group_max<LPT>(cm);
-      const float m_new = fmaxf(m_run[h], cm);
-      const float alpha = fast_exp2(m_run[h] - m_new);
-      m_run[h] = m_new;
-      l_run[h] *= alpha;
+    for (int e = 0; e < 4 * VC; ++e) acc[e] *= alpha;
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) acc[h][e] *= alpha;
-    }
+    for (int j = 0; j < 4; ++j) {
+      const float p = fast_exp2(s[j] - m);
+      l += p;
+      const bool seen = vpos + j < p1;     // what stands in for a row past the context counts as zeros
 #pragma unroll
-    for (int i = 0; i < CH_LOADS; ++i) {
+      for (int c = 0; c < VC; ++c)
 #pragma unroll
-      for (int h = 0; h < REP; ++h) {
-        const float p = fast_exp2(s[i][h] - m_run[h]);
-        l_run[h] += p;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[h][e] = fmaf(p, bits_to_f32(vbuf[i].w[e]), acc[h][e]);
-      }
+        for (int i = 0; i < 4; ++i)
+          acc[4 * c + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(seen ? bits_to_f32(v[j][c].w[i]) : 0.f, p,
+                                                                acc[4 * c + i], 0, 0, 0);
     }
   }
+  l = sum_xor32(sum_xor16(l));
 
-  // l was accumulated per token slot; sum over the slots like acc
+  // ---- merge the waves ----
+  float2* const ml = reinterpret_cast<float2*>(f32_lds + NW * R * S::PITCH);   // [wave][16]
+  if (lg == 0) ml[16 * wave + lc] = make_float2(m, l);
+  __syncthreads();
+  const int busy = min(NW, (p1 - p0 + 15) >> 4);       // waves that saw a position
+  if (lc < R && wave < busy) {
+    float M = m;
+    for (int w = 0; w < busy; ++w) M = max_f32(M, ml[16 * w + lc].x);
+    const float f = fast_exp2(m - M);
+    float* const dst = f32_lds + (wave * R + lc) * S::PITCH + 16 * lg;
 #pragma unroll
-  for (int h = 0; h < REP; ++h) {
-    l_run[h] = cross_group_sum<LPT>(l_run[h]);
+    for (int c = 0; c < VC; ++c)
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) acc[h][e] = cross_group_sum<LPT>(acc[h][e]);
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<float4_t*>(dst + 64 * c + 4 * j) =
+            float4_t{acc[4 * c][j], acc[4 * c + 1][j], acc[4 * c + 2][j], acc[4 * c + 3][j]} * f;
   }
-  finish_valu<Tag, D, REP, EPL, LPT>(a, row, part, head0, lane, acc, m_run, l_run);
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < R * (D / 4); idx += 64 * NW) {
+    const int h = idx / (D / 4), d4 = idx - h * (D / 4), head = head0 + h;
+    float M = ml[h].x;
+    for (int w = 1; w < busy; ++w) M = max_f32(M, ml[16 * w + h].x);
+    float L = 0.f, L2 = 0.f;                 // even and odd waves apart: shorter chains of sums
+    float4_t o = float4_t{0.f, 0.f, 0.f, 0.f}, o2 = o;
+    for (int w = 0; w < busy; w += 2) {
+      const float2 x = ml[16 * w + h];
+      L = fmaf(x.y, fast_exp2(x.x - M), L);
+      o += *reinterpret_cast<const float4_t*>(f32_lds + (w * R + h) * S::PITCH + 4 * d4);
+      if (w + 1 < busy) {
+        const float2 y = ml[16 * (w + 1) + h];
+        L2 = fmaf(y.y, fast_exp2(y.x - M), L2);
+        o2 += *reinterpret_cast<const float4_t*>(f32_lds + ((w + 1) * R + h) * S::PITCH + 4 * d4);
+      }
+    }
+    L += L2;
+    o += o2;
+    if (nparts == 1) {
+      st_through(a.out + row * a.out_row_bytes + ((int64_t)head * D + 4 * d4) * 4, o * (1.f / L));
+    } else {
+      const int64_t pidx = (int64_t)(pbeg + part) * a.num_heads + head;
+      *reinterpret_cast<float4_t*>(a.ws_acc + pidx * D + 4 * d4) = o;
+      if (d4 == 0) *reinterpret_cast<float2*>(a.ws_ml + pidx * 2) = make_float2(M, L);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1108,25 +1103,24 @@ __global__ __launch_bounds__(COMBINE_THREADS) void combine_partials_kernel(const
 }
 
 // ---- dispatch ---------------------------------------------------------------
-template <typename Tag, int D, int REP>
-static void launch_valu(const attn_args& a, int num_work, hipStream_t stream) {
-  hipLaunchKernelGGL((paged_attn_valu_kernel<Tag, D, REP>), dim3(num_work, a.num_kv_heads, a.rep / a.group),
-                     dim3(64), 0, stream, a);
+template <int D, int NW>
+static void launch_f32_nw(const attn_args& a, int num_work, hipStream_t stream) {
+  using S = f32_shape<D, NW>;
+  const size_t lds = (size_t)NW * (a.group * S::PITCH + 32) * sizeof(float);
+  hipLaunchKernelGGL((paged_attn_f32_kernel<D, NW>), dim3(num_work, a.num_kv_heads, a.rep / a.group), dim3(64 * NW), lds,
+                     stream, a);
 }
 
+// A step of few work items is a chain of latencies: a whole partition in flight (16 waves; 8
+// at head dim 128, whose registers do not fit 16). From 256 workgroups on (one per CU)
+// four waves: more workgroups on a CU hide the chain better than more waves on an item.
 template <int D>
-static int dispatch_valu_rep(const attn_args& a, int num_work, hipStream_t s) {
-  switch (a.group) {
-    case 1: launch_valu<f32_t, D, 1>(a, num_work, s); return TB_OK;
-    case 2: launch_valu<f32_t, D, 2>(a, num_work, s); return TB_OK;
-    case 3: launch_valu<f32_t, D, 3>(a, num_work, s); return TB_OK;
-    case 4: launch_valu<f32_t, D, 4>(a, num_work, s); return TB_OK;
-    case 5: launch_valu<f32_t, D, 5>(a, num_work, s); return TB_OK;
-    case 6: launch_valu<f32_t, D, 6>(a, num_work, s); return TB_OK;
-    case 7: launch_valu<f32_t, D, 7>(a, num_work, s); return TB_OK;
-    case 8: launch_valu<f32_t, D, 8>(a, num_work, s); return TB_OK;
-    default: return TB_ERR_UNSUPPORTED;
-  }
+static void launch_f32(const attn_args& a, int num_work, hipStream_t stream) {
+  if (num_work <= 0) return;
+  if ((int64_t)num_work * a.num_kv_heads * (a.rep / a.group) < 256)
+    launch_f32_nw<D, D == 64 ? 16 : 8>(a, num_work, stream);
+  else
+    launch_f32_nw<D, 4>(a, num_work, stream);
 }
 
 template <typename Tag, int D>
@@ -1298,8 +1292,8 @@ static int32_t paged_attention_impl(const void* q, int64_t q_row_stride, void* p
   }
 
   const int rep = num_heads / num_kv_heads;
-  // heads per wave: the MFMA operand holds 16; the fp32 kernel keeps 8 in registers
-  const int group = largest_divisor_upto(rep, eb == 2 ? 16 : 8);
+  // heads per workgroup: the MFMA operand holds 16; the fp32 kernel's merge keeps to 64 KiB of LDS
+  const int group = largest_divisor_upto(rep, eb == 2 ? 16 : head_dim == 64 ? 14 : 7);
   const bool merged = slot_map != nullptr;
   if (merged) {   // split rows merged inside the launch of the 16-bit work-item kernel
     if (eb != 2 || num_prefill_tiles > 0 || group != rep || device_counts) return TB_ERR_UNSUPPORTED;
@@ -1362,12 +1356,10 @@ static int32_t paged_attention_impl(const void* q, int64_t q_row_stride, void* p
     }
     TB_RETURN_LAUNCH_STATUS();
   }
-  int st = TB_OK;
   switch (dtype) {
     case TB_DTYPE_F32:
-      st = d64 ? dispatch_valu_rep<64>(a, num_work_items, stream) : dispatch_valu_rep<128>(a, num_work_items, stream);
-      if (st == TB_OK)
-        d64 ? launch_combine<f32_t, 64>(a, num_split_rows, stream) : launch_combine<f32_t, 128>(a, num_split_rows, stream);
+      d64 ? launch_f32<64>(a, num_work_items, stream) : launch_f32<128>(a, num_work_items, stream);
+      d64 ? launch_combine<f32_t, 64>(a, num_split_rows, stream) : launch_combine<f32_t, 128>(a, num_split_rows, stream);
       break;
     case TB_DTYPE_F16:
       launch_16bit<f16_t>(a, d64, num_work_items, num_prefill_tiles, num_split_rows, stream);
@@ -1377,7 +1369,6 @@ static int32_t paged_attention_impl(const void* q, int64_t q_row_stride, void* p
       break;
     default: return TB_ERR_INVALID_ARG;
   }
-  if (st != TB_OK) return st;
   TB_RETURN_LAUNCH_STATUS();
 }
 

@@ -349,6 +349,7 @@ __global__ __launch_bounds__(64 * cshape<D>::NW, 2) void paged_prefill_columns_k
   if (!mine) return;
   const int row = row0 + my_row;
   const int pbeg = a.row_part_off[row], nparts = a.row_part_off[row + 1] - pbeg;
+  if (part >= nparts) return;                   // the row ends before this part
   if (nparts == 1) {                            // the whole row: final output
     const float inv = 1.f / l;
     char* const orow = a.out + (int64_t)row * a.out_row_bytes + (int64_t)hd * RB + 8 * half;
@@ -362,7 +363,212 @@ __global__ __launch_bounds__(64 * cshape<D>::NW, 2) void paged_prefill_columns_k
         for (int j = 0; j < 4; ++j) o[j] = (scalar_t)(acc[b][4 * g + j] * inv);
         st8_through(orow + 64 * b + 16 * g, o);
       }
-  } else if (part < nparts) {                   // partial of a split row (rows ending before the part own no slot)
+  } else {                                      // partial of a split row
+    const int64_t slot_i = (int64_t)(pbeg + part) * a.num_heads + hd;
+    float* const dst = a.ws_acc + slot_i * D + 4 * half;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4_t*>(dst + 32 * b + 8 * g) =
+            float4_t{acc[b][4 * g], acc[b][4 * g + 1], acc[b][4 * g + 2], acc[b][4 * g + 3]};
+    if (half == 0) *reinterpret_cast<float2*>(a.ws_ml + slot_i * 2) = make_float2(m, l);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The same work in fp32: v_mfma_f32_32x32x2_f32 (fp32 products and sums), chunks of
+// 32 positions. k index half of a product stands for dim 8 c + 4 half + i of the K rows and
+// q (whole 16-byte loads, component by component), and for position 8 (r / 4) + 4 half +
+// r % 4 of V and P, whose B operand is then register r of the scores as it is. A
+// score's dims are summed in eight chains, and a chunk's P.V apart from the chunks before
+// it, so that rounding stays at the level of the row-by-row kernel's (distance from 64-bit
+// results 1.4e-7; 2.2e-7 with two chains and one running sum).
+//
+// Bound by the fp32 matrix rate (154 TFLOP/s for a library product here). us per
+// layer for six prompts of 201..687 tokens at 14 / 2 heads of 64: 59 with the append, against
+// 119 for one work item per row.
+template <int D>
+struct fshape {
+  static constexpr int RB = 4 * D;
+  static constexpr int TB = 16 * RB;
+  static constexpr int CK = 32;                 // positions per chunk
+  static constexpr int HALF = CK * RB;
+  static constexpr int SLOT = 2 * HALF;
+  static constexpr int PPR = RB / 16;           // 16-byte pieces per row
+  static constexpr int RPL = 64 / PPR;          // rows per direct load
+  static constexpr int TLD = TB / 1024;
+  static constexpr int KC = D / 8;              // 16-byte K chunks of a lane
+  static constexpr int NB = D / 32;
+  // 16 lanes of a K read touch 16 rows of one piece: spread over the 16 pieces of 64 banks
+  static __device__ __forceinline__ int kswz(int r) { return r & 15; }
+};
+
+template <int D>
+__global__ __launch_bounds__(256, D == 64 ? 2 : 1) void paged_prefill_columns_f32_kernel(const cols_args a) {
+  using S = fshape<D>;
+  constexpr int RB = S::RB, TB = S::TB, CK = S::CK, KC = S::KC, NB = S::NB, COLS_ = 128;
+  extern __shared__ __align__(1024) char flds[];   // two chunks
+
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, lcol = lane & 31, half = lane >> 5;
+  const int4 w0 = a.work[2 * blockIdx.x], w1 = a.work[2 * blockIdx.x + 1];
+  const int row0 = w0.x, seq = w0.y, pos0 = w0.z, nrows = w0.w;
+  if (nrows == 0) return;                       // a padding entry (whole workgroup)
+  const int col0 = w1.x, kvh = w1.y, part = w1.z, part_chunks = 2 * w1.w;   // the list counts chunks of 64
+  const int rep = a.rep, ncols = nrows * rep;
+  const int col = col0 + 32 * wave + lcol;
+  const bool mine = col < ncols;
+  const int ccol = mine ? col : ncols - 1;
+  const int my_row = ccol / rep, hd = kvh * rep + ccol - my_row * rep;
+  const int my_pos = pos0 + my_row;
+  const int wcol = min(col0 + 32 * wave, ncols - 1);
+  const bool wave_busy = col0 + 32 * wave < ncols;
+  const int wave_first = pos0 + wcol / rep;
+  const int wave_last = pos0 + min(col0 + 32 * wave + 31, ncols - 1) / rep;
+  const int limit = pos0 + min(col0 + COLS_ - 1, ncols - 1) / rep + 1;
+  const int c_begin = part * part_chunks;
+  const int c_end = min(c_begin + part_chunks, (limit + CK - 1) / CK);
+
+  vec16 q[KC];                                  // dims 8 c + 4 half .. of the column
+  {
+    const char* qrow = a.q + (int64_t)(row0 + my_row) * a.q_row_bytes + (int64_t)hd * RB + 16 * half;
+#pragma unroll
+    for (int c = 0; c < KC; ++c) q[c] = ld16(qrow + 32 * c);
+  }
+  // ---- direct loads: a chunk's K tiles by waves 0, 1 and its V tiles by waves 2, 3 ----
+  const int64_t head_bytes = ((int64_t)1 << a.log2_bs) * RB;
+  const int64_t blk_bytes = 2 * (int64_t)a.num_kv_heads * head_bytes;
+  const int64_t v_off = a.num_kv_heads * head_bytes;
+  const int sub_mask = (1 << (a.log2_bs - 4)) - 1;
+  const int32_t* const table = a.block_tables + (int64_t)seq * a.max_nb;
+  const int last_tile = (limit - 1) >> 4;
+  const int lt = wave & 1;
+  const bool is_v = wave >= 2;
+  const char* const pool_src = a.pool + kvh * head_bytes + (is_v ? v_off : 0);
+  const int lrow = lane / S::PPR, lpiece = lane % S::PPR;
+  int id0 = c_begin;
+  auto load_ids = [&](int c) {                  // lane j: the block of this wave's tile in chunk c + j
+    const int t = min(2 * (c + lane) + lt, last_tile);
+    int b = table[(t << 4) >> a.log2_bs];
+    return (b < 0 || b >= a.num_blocks) ? 0 : b;   // host validates; stay inside the pool
+  };
+  int ids = load_ids(id0);
+  auto issue = [&](int c, int slot) {
+    if (c - id0 >= 64) {
+      id0 = c;
+      ids = load_ids(id0);
+    }
+    const int t = min(2 * c + lt, last_tile);
+    const int rmax = limit - 1 - 16 * t;
+    const int64_t b = __builtin_amdgcn_readlane(ids, c - id0);
+    const char* const base = pool_src + b * blk_bytes + (int64_t)(t & sub_mask) * TB;
+    char* const dst = flds + slot * S::SLOT + (is_v ? S::HALF : 0) + lt * TB;
+#pragma unroll
+    for (int i = 0; i < S::TLD; ++i) {
+      const int r = S::RPL * i + lrow;
+      s_dma16_l2((uint32_t)(min(r, rmax) * RB + 16 * (is_v ? lpiece : lpiece ^ S::kswz(r))), base, dst + 1024 * i);
+    }
+  };
+  asm volatile("" : "+v"(ids));
+  if (c_begin < c_end) issue(c_begin, 0);
+  if (a.rope.cos) {                             // chunk c pairs with chunk c + KC/2 (dims i and i + D/2)
+    const int64_t r = a.rope.row(my_pos, D / 2) + 4 * half;
+#pragma unroll
+    for (int c = 0; c < KC / 2; ++c)
+      rope_pair<float>(q[c], q[c + KC / 2], a.rope.cos + r + 8 * c, a.rope.sin + r + 8 * c);
+  }
+#pragma unroll
+  for (int c = 0; c < KC; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(q[c].w[i]));
+
+  float m = -INFINITY, l = 0.f;
+  float16_t acc[NB];                            // O^T[32 b + 8 (r / 4) + 4 half + r % 4][col]
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
+  const float sl2e = a.scale_log2e;
+  const int n = c_end - c_begin;
+  const int n_wave = wave_busy ? min(c_end - 1, wave_last / CK) - c_begin + 1 : 0;
+  for (int k = 0; k < n; ++k) {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // as the 16-bit kernel
+    if (k + 1 < n) issue(c_begin + k + 1, (k + 1) & 1);
+    if (k >= n_wave) continue;
+    const int c = c_begin + k;
+    const char* const base = flds + (k & 1) * S::SLOT;
+    float16_t sh[2];                            // chains of 8 dims (D / 8 at head dim 128), added pairwise
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float16_t d4[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) d4[i][r] = 0.f;
+#pragma unroll
+      for (int cc = h * KC / 2; cc < (h + 1) * KC / 2; ++cc) {
+        const vec16 kv = ld16(base + lcol * RB + 16 * ((2 * cc + half) ^ S::kswz(lcol)));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          d4[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(bits_to_f32(kv.w[i]), bits_to_f32(q[cc].w[i]), d4[i], 0, 0, 0);
+      }
+      sh[h] = (d4[0] + d4[1]) + (d4[2] + d4[3]);
+    }
+    float16_t sc = sh[0] + sh[1];
+    if (CK * c + CK - 1 > wave_first) {         // the chunk crosses the diagonal of some column
+      asm volatile("");
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (CK * c + 8 * (r >> 2) + 4 * half + (r & 3) > my_pos) sc[r] = -INFINITY;
+    }
+    float cm = max_f32(sc[0], sc[1]);
+#pragma unroll
+    for (int e = 2; e < 16; e += 2) cm = max3_f32(cm, sc[e], sc[e + 1]);
+    cm = max_xor32(cm) * sl2e;
+    if (__any(cm > m)) {
+      const float m_new = fmaxf(m, cm);
+      const float alpha = fast_exp2(m - (m_new == -INFINITY ? 0.f : m_new));   // 0 while m = -inf
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[b] *= alpha;
+    }
+    const float m_safe = m == -INFINITY ? 0.f : m;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sc[r] = fast_exp2(sc[r] * sl2e - m_safe);
+    l += (((sc[0] + sc[1]) + (sc[2] + sc[3])) + ((sc[4] + sc[5]) + (sc[6] + sc[7]))) +
+         (((sc[8] + sc[9]) + (sc[10] + sc[11])) + ((sc[12] + sc[13]) + (sc[14] + sc[15])));
+    const char* const vb = base + S::HALF + 4 * half * RB + 4 * lcol;
+    float16_t pv[NB];                           // the chunk's own sum: shorter chains than one over all positions
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) pv[b][r] = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        pv[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+            *reinterpret_cast<const float*>(vb + (8 * (r >> 2) + (r & 3)) * RB + 128 * b), sc[r], pv[b], 0, 0, 0);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[b] += pv[b];
+  }
+
+  l = sum_xor32(l);
+  if (!mine) return;
+  const int row = row0 + my_row;
+  const int pbeg = a.row_part_off[row], nparts = a.row_part_off[row + 1] - pbeg;
+  if (part >= nparts) return;                   // the row ends before this part
+  if (nparts == 1) {
+    const float inv = 1.f / l;
+    char* const orow = a.out + (int64_t)row * a.out_row_bytes + (int64_t)hd * RB + 16 * half;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        st_through(orow + 128 * b + 32 * g, float4_t{acc[b][4 * g], acc[b][4 * g + 1], acc[b][4 * g + 2], acc[b][4 * g + 3]} * inv);
+  } else {
     const int64_t slot_i = (int64_t)(pbeg + part) * a.num_heads + hd;
     float* const dst = a.ws_acc + slot_i * D + 4 * half;
 #pragma unroll
@@ -516,14 +722,15 @@ extern "C" int32_t tb_paged_prefill_columns(const void* q, int64_t q_row_stride,
   TB_CHECK_ARG(num_work >= 0 && num_rows >= 0 && num_split_rows >= 0 && num_split_rows <= num_rows);
   TB_CHECK_ARG(num_heads > 0 && num_kv_heads > 0 && num_heads % num_kv_heads == 0);
   if (num_work == 0) return TB_OK;
-  if (dtype != TB_DTYPE_F16 && dtype != TB_DTYPE_BF16) return TB_ERR_UNSUPPORTED;
+  const int eb = dtype == TB_DTYPE_F32 ? 4 : dtype == TB_DTYPE_F16 || dtype == TB_DTYPE_BF16 ? 2 : 0;
+  TB_CHECK_ARG(eb > 0);
   if (head_dim != 64 && head_dim != 128) return TB_ERR_UNSUPPORTED;
   if (block_size < 16 || (block_size & (block_size - 1))) return TB_ERR_UNSUPPORTED;
   TB_CHECK_ARG(q && pool && out && block_tables && work && row_part_offsets && num_rows > 0);
   TB_CHECK_ARG(num_blocks > 0 && max_blocks_per_seq > 0 && max_parts_per_row >= 0 && total_partitions >= 0);
   TB_CHECK_ARG(q_row_stride >= (int64_t)num_heads * head_dim && out_row_stride >= (int64_t)num_heads * head_dim);
   TB_CHECK_ARG((((uintptr_t)q | (uintptr_t)pool | (uintptr_t)out | (uintptr_t)work) & 15u) == 0);
-  TB_CHECK_ARG((q_row_stride * 2) % 16 == 0 && (out_row_stride * 2) % 16 == 0);
+  TB_CHECK_ARG((q_row_stride * eb) % 16 == 0 && (out_row_stride * eb) % 16 == 0);
   TB_CHECK_ARG(num_split_rows == 0 || (split_rows && max_parts_per_row > 1));
   TB_CHECK_ARG(((uintptr_t)split_rows & 15u) == 0);
   TB_CHECK_ARG(!rope_cos == !rope_sin && (!rope_cos || rope_max_position > 0));
@@ -542,11 +749,11 @@ extern "C" int32_t tb_paged_prefill_columns(const void* q, int64_t q_row_stride,
   }
   cols_args a{};
   a.q = static_cast<const char*>(q);
-  a.q_row_bytes = q_row_stride * 2;
+  a.q_row_bytes = q_row_stride * eb;
   a.pool = static_cast<const char*>(pool);
   a.num_blocks = num_blocks;
   a.out = static_cast<char*>(out);
-  a.out_row_bytes = out_row_stride * 2;
+  a.out_row_bytes = out_row_stride * eb;
   a.block_tables = block_tables;
   a.max_nb = max_blocks_per_seq;
   a.work = reinterpret_cast<const int4*>(work);
@@ -561,7 +768,10 @@ extern "C" int32_t tb_paged_prefill_columns(const void* q, int64_t q_row_stride,
   a.rope = rope_tables{rope_cos, rope_sin, rope_max_position};
   const dim3 grid(num_work), block(64 * cshape<64>::NW);
   const bool d64 = head_dim == 64;
-  if (dtype == TB_DTYPE_F16) {
+  if (dtype == TB_DTYPE_F32) {
+    if (d64) hipLaunchKernelGGL((paged_prefill_columns_f32_kernel<64>), grid, block, 2 * fshape<64>::SLOT, stream, a);
+    else hipLaunchKernelGGL((paged_prefill_columns_f32_kernel<128>), grid, block, 2 * fshape<128>::SLOT, stream, a);
+  } else if (dtype == TB_DTYPE_F16) {
     if (d64) hipLaunchKernelGGL((paged_prefill_columns_kernel<f16_t, 64>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((paged_prefill_columns_kernel<f16_t, 128>), grid, block, 0, stream, a);
   } else {
@@ -569,7 +779,7 @@ extern "C" int32_t tb_paged_prefill_columns(const void* q, int64_t q_row_stride,
     else hipLaunchKernelGGL((paged_prefill_columns_kernel<bf16_t, 128>), grid, block, 0, stream, a);
   }
   if (num_split_rows > 0)
-    combine_split_rows(dtype, head_dim, num_heads, out, out_row_stride * 2, split_rows, num_split_rows, a.ws_acc, a.ws_ml,
+    combine_split_rows(dtype, head_dim, num_heads, out, out_row_stride * eb, split_rows, num_split_rows, a.ws_acc, a.ws_ml,
                        stream);
   TB_RETURN_LAUNCH_STATUS();
 }

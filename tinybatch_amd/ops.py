@@ -271,14 +271,14 @@ def columns_route(dtype: torch.dtype, num_heads: int, num_kv_heads: int, head_di
                   device: torch.device):
     """The ColumnsRoute (build_step_metadata's columns_route) that sends prefill sequences of
     any context to tb_paged_prefill_columns for this geometry, or None where that kernel
-    does not serve it (fp32, other head dims, blocks of fewer than 16 positions).
+    does not serve it (other head dims, blocks of fewer than 16 positions).
 
     Against the 64-row tiles it replaces (bf16, us per layer): four prompts of 1746..3738
     tokens at 14 / 2 heads of 64: 90 against 135; three of 5300..7333 at 32 / 8 heads of
     128: 1070 against 3550."""
     from .metadata import ColumnsRoute
 
-    if (dtype not in (torch.float16, torch.bfloat16) or num_kv_heads <= 0 or num_heads % num_kv_heads
+    if (dtype not in _lib.DTYPE_CODE or num_kv_heads <= 0 or num_heads % num_kv_heads
             or head_dim not in (64, 128) or block_size < 16 or block_size & (block_size - 1)):
         return None
     d = decode_device(device)
