@@ -202,3 +202,24 @@ def test_norm_kernels_agree_bit_for_bit(dtype):
         b = layer_ops.rms_norm_partials(x.float()[None].contiguous(), w, 1e-6, residual=rb)
         assert torch.equal(ra, rb)
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), rows
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,dim,pad", [(1, 8, 0), (5, 512, 8), (3, 1024, 0), (7, 2056, 8), (2, 896, 1)])
+def test_norm_and_gate_chunked_and_plain_rows(dtype, rows, dim, pad):
+    """Rows of whole aligned 16-byte chunks take the chunked kernels, others (pad 1) the plain
+    ones: either against the oracle's functions, and the gate bit for bit between the two."""
+    g = torch.Generator().manual_seed(rows * dim + pad)
+    x = torch.randn(rows, 2 * dim + pad, generator=g).to(dtype).to(DEV)
+    w = (1 + 0.1 * torch.randn(dim, generator=g)).to(dtype).to(DEV)
+    res = torch.randn(rows, dim + pad, generator=g).to(dtype).to(DEV)[:, :dim]
+    h = res.cpu() + x[:, :dim].cpu()
+    got = layer_ops.rms_norm(x[:, :dim], w, 1e-6, residual=res)
+    assert torch.equal(res.cpu(), h)
+    torch.testing.assert_close(got.cpu().float(), mref.rms_norm(h, w.cpu(), 1e-6).float(), **TOL[dtype])
+    got = layer_ops.silu_mul(x, dim)
+    want = F.silu(x[:, :dim].cpu()) * x[:, dim:2 * dim].cpu()
+    torch.testing.assert_close(got.cpu().float(), want.float(), **TOL[dtype])
+    odd = torch.empty(rows, 2 * dim + 1, dtype=dtype, device=DEV)   # an odd row stride: the plain kernel
+    odd[:, :2 * dim] = x[:, :2 * dim]
+    assert torch.equal(layer_ops.silu_mul(odd, dim), got)
