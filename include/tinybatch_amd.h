@@ -275,9 +275,11 @@ int32_t tb_paged_prefill_columns(const void* q, int64_t q_row_stride, const void
                                  hipStream_t stream);
 /* The partition length (positions, a multiple of 64) for a step's sequences of new_rows new
  * rows from position pos0 on a GPU of num_cus CUs: longer than every context unless the
- * step has too few rows to keep the CUs busy. Negative: a status code. */
+ * step has too few rows to keep the CUs busy. other_partitions: the partitions of the
+ * step's other rows, which share the partials' workspace. Negative: a status code. */
 int32_t tb_prefill_columns_partition(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs,
-                                     int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t num_cus);
+                                     int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t dtype,
+                                     int32_t num_cus, int32_t other_partitions);
 /* The work list (host, no device call): *count entries of 8 int32 into work (work NULL: the
  * count alone). Entry g is meant for XCD g % num_xcds (1: placement unknown). */
 int32_t tb_build_prefill_columns_work(const int32_t* first_row, const int32_t* seq_index, const int32_t* pos0,

@@ -39,10 +39,15 @@ def test_every_row_head_and_partition_once(hq, hkv, xcds, part):
 def test_partitions():
     r = ColumnsRoute(14, 2, 64, 8, 256)
     assert columns_partition([0] * 4, [3251, 1746, 3738, 2168], r) > 3738         # enough rows: none split
+    assert columns_partition([0], [600], r) >= 600                              # a merge would cost more than it saves
     p = columns_partition([3000] * 4, [20] * 4, r)
-    assert p % 64 == 0 and p <= TILE_PARTITION
-    p = columns_partition([9000], [1500], r)                                    # the scratch bound
-    assert p == TILE_PARTITION
+    assert p % 64 == 0 and p < TILE_PARTITION
+    # a call without a workspace: shorter than the tiles' partition only within the static scratch
+    slot = 14 * 66 * 4
+    for pos0, n, other in ((9000, 1500, 0), (1000, 100, 0), (1000, 100, (32 << 20) // slot)):
+        p = columns_partition([pos0], [n], r, other)
+        slots = other + sum(-(-(pos0 + i + 1) // p) for i in range(n))
+        assert p >= TILE_PARTITION or slots * slot <= 32 << 20
     with pytest.raises(RuntimeError):
         columns_partition([0], [0], r)
 

@@ -615,9 +615,11 @@ int columns_limit(int pos0, int new_rows, int rep, int col0) {
 
 extern "C" int32_t tb_prefill_columns_partition(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs,
                                                 int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
-                                                int32_t num_cus) {
-  if (!columns_args_ok(pos0, new_rows, num_seqs, num_heads, num_kv_heads) || num_cus <= 0) return TB_ERR_INVALID_ARG;
-  if (head_dim != 64 && head_dim != 128) return TB_ERR_INVALID_ARG;
+                                                int32_t dtype, int32_t num_cus, int32_t other_partitions) {
+  if (!columns_args_ok(pos0, new_rows, num_seqs, num_heads, num_kv_heads) || num_cus <= 0 || other_partitions < 0)
+    return TB_ERR_INVALID_ARG;
+  if ((head_dim != 64 && head_dim != 128) || (dtype != TB_DTYPE_F32 && dtype != TB_DTYPE_F16 && dtype != TB_DTYPE_BF16))
+    return TB_ERR_INVALID_ARG;
   const int rep = num_heads / num_kv_heads;
   int64_t total = 0;
   int longest = 0;
@@ -627,20 +629,40 @@ extern "C" int32_t tb_prefill_columns_partition(const int32_t* pos0, const int32
       total += (int64_t)n * num_kv_heads;
       longest = std::max(longest, n);
     }
-  const int whole = (longest + 1) * CHUNK;             // no row is split
-  const int64_t share = (total + num_cus - 1) / num_cus;   // chunks per CU
-  if (longest <= share) return whole;
-  // the scratch a split needs (partials of every row that is longer than a partition)
-  auto scratch = [&](int64_t part) {
-    int64_t parts = 0;
-    for (int i = 0; i < num_seqs; ++i)
-      for (int r = 0; r < new_rows[i]; ++r) parts += (pos0[i] + r + part) / part;
-    return parts * num_heads * (head_dim + 2) * 4;
-  };
-  int part = std::max(8, (int)((share + 1) / 2));
-  part = std::min(part, 16);
-  if (part < 16 && scratch((int64_t)part * CHUNK) > TB_NOALLOC_SCRATCH_BYTES) part = 16;
-  return part * CHUNK < whole ? part * CHUNK : whole;
+  // The partition with the least cost, in us: a workgroup alone on its CU takes 1.0 (head
+  // dim 64) or 1.6 us a chunk, a full CU 0.65 or 1.05 us per chunk of its workgroups (fp32, at
+  // the matrix rate either way: 4 or 8 and 3.6 or 7.2); a split
+  // adds the merge's launch (5 us) and its rows' partials, written and read (4 bytes/ps).
+  // Measured in a graph with the append, bf16, 14 / 2 heads of 64, us per layer: 16 prefix hits
+  // of 100 rows after 3008 positions 41.4 (45.4 when split at 512 positions), 4 of 30 after
+  // 704 14.2 (16.9), one fresh prompt of 600 unsplit 16.8 (17.7).
+  const bool d64 = head_dim == 64, f32 = dtype == TB_DTYPE_F32;
+  const double alone = f32 ? (d64 ? 4.0 : 8.0) : d64 ? 1.0 : 1.6, full = f32 ? (d64 ? 3.6 : 7.2) : d64 ? 0.65 : 1.05;
+  const double share = full * (double)total / num_cus;
+  auto span = [&](int chunks) { return std::max(alone * chunks, share + 0.5 * full * chunks); };
+  int best = longest + 1;                              // longer than every context: no row is split
+  double cost = span(longest);
+  for (int part = 4; part < longest; part += part < 16 ? 2 : part < 64 ? 8 : 32) {
+    const int64_t tokens = (int64_t)part * CHUNK;
+    int64_t parts = 0, slots = other_partitions;       // partials of split rows; partitions of all rows
+    for (int i = 0; i < num_seqs; ++i) {
+      // rows of k partitions: positions (k - 1) tokens .. k tokens - 1
+      const int64_t first = pos0[i], last = first + new_rows[i];
+      for (int64_t k = first / tokens + 1; (k - 1) * tokens < last; ++k) {
+        const int64_t rows_k = std::min(last, k * tokens) - std::max(first, (k - 1) * tokens);
+        slots += k * rows_k;
+        if (k > 1) parts += k * rows_k;
+      }
+    }
+    const double slot_bytes = (double)num_heads * (head_dim + 2) * 4;
+    // a call without a workspace still finds room: shorter than the tiles' 1024 positions only
+    // while the step's partials fit the static scratch
+    if (part < 16 && slots * slot_bytes > TB_NOALLOC_SCRATCH_BYTES) continue;
+    // the merge reads eight partials at a time: each eight more are another round trip
+    const double c = span(part) + 5.0 + 3.0 * ((longest - 1) / part / 8) + 2 * parts * slot_bytes / 4e6;
+    if (c < 0.95 * cost) cost = c, best = part;
+  }
+  return best * CHUNK;
 }
 
 extern "C" int32_t tb_build_prefill_columns_work(const int32_t* first_row, const int32_t* seq_index, const int32_t* pos0,

@@ -221,7 +221,8 @@ class PrefillRoute(NamedTuple):
 
 class ColumnsRoute(NamedTuple):
     """Where prefill sequences of any context go to tb_paged_prefill_columns in place of
-    tiles: the step's heads and head dim, the GPU's XCDs and CUs (ops.columns_route)."""
+    tiles and fp32 work items: the step's heads, head dim and element type (the C ABI's
+    code), the GPU's XCDs and CUs (ops.columns_route)."""
     num_heads: int
     num_kv_heads: int
     head_dim: int
@@ -237,13 +238,16 @@ def _i32_columns(*columns):
     return cols, [c.ctypes.data_as(ctypes.c_void_p) for c in cols]
 
 
-def columns_partition(pos0s, new_rows, route: ColumnsRoute) -> int:
-    """tb_prefill_columns_partition: positions per partition of the step's column rows."""
+    dtype: int = 2
+def columns_partition(pos0s, new_rows, route: ColumnsRoute, other_partitions: int = 0) -> int:
+    """tb_prefill_columns_partition: positions per partition of the step's column rows
+    (``other_partitions``: those of its other rows)."""
     from . import _lib
 
     cols, ptrs = _i32_columns(pos0s, new_rows)
     p = int(_lib.lib().tb_prefill_columns_partition(*ptrs, cols[0].size, route.num_heads, route.num_kv_heads,
-                                                    route.head_dim, route.num_cus))
+                                                    route.head_dim, route.dtype, route.num_cus,
+                                                    other_partitions))
     if p < 0:
         _lib.check(p, "tb_prefill_columns_partition")
     return p
@@ -415,7 +419,6 @@ def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, bl
                 if n >= 16 and not tiled[int(starts[b])]:
                     column_seqs.append((int(starts[b]), b, c - n, n))
             if column_seqs:
-                part = columns_partition([x[2] for x in column_seqs], [x[3] for x in column_seqs], columns_route)
                 for s0, _, _, n in column_seqs:
                     tiled[s0:s0 + n] = True               # served by tb_paged_prefill_columns
                     nparts_by_row[s0:s0 + n] = (row_ctx_by_row[s0:s0 + n] + part - 1) // part
@@ -428,6 +431,9 @@ def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, bl
                     tiled[s0:s0 + n] = True               # served by tiles, not work items
                     rc = row_ctx_by_row[s0:s0 + n]
                     nparts_by_row[s0:s0 + n] = (rc + TILE_PARTITION - 1) // TILE_PARTITION
+                part = columns_partition([x[2] for x in column_seqs], [x[3] for x in column_seqs], columns_route,
+                                         int(nparts_by_row[~tiled].sum()))
+                for s0, _, _, n in column_seqs:
                     for r in range(0, n, TILE_ROWS):
                         rows = min(TILE_ROWS, n - r)
                         pos0 = c - n + r

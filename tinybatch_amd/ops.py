@@ -282,7 +282,8 @@ def columns_route(dtype: torch.dtype, num_heads: int, num_kv_heads: int, head_di
             or head_dim not in (64, 128) or block_size < 16 or block_size & (block_size - 1)):
         return None
     d = decode_device(device)
-    return ColumnsRoute(num_heads, num_kv_heads, head_dim, d.num_xcds if d.merge_in_kernel else 1, d.workgroups)
+    return ColumnsRoute(num_heads, num_kv_heads, head_dim, d.num_xcds if d.merge_in_kernel else 1, d.workgroups,
+                        _lib.DTYPE_CODE[dtype])
 
 
 def decode_kernel_preferred(meta: StepMetadata, *, num_kv_heads: int, head_dim: int, dtype: torch.dtype,
