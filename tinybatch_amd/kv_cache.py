@@ -199,8 +199,7 @@ class PagedKVCache:
 
     @staticmethod
     def _fusable(meta: StepMetadata) -> bool:
-        sm = meta.slot_mapping_np
-        if sm.size and np.any((sm < 0) & (meta.row_ctx_np > 0)):
+        if meta.has_superseded():
             return False                                  # a superseded writer: the separate append
         if meta.parts is not None or meta.decode_only:
             return True

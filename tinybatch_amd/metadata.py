@@ -115,6 +115,16 @@ class StepMetadata:
     # still describe the whole step (its slot mapping serves the append)
     parts: list | None = None
 
+    # whether a row's slot is also written by a later row of the step (its slot_mapping is
+    # -1): no fused append then. Found by the builder; None: found from the arrays when asked
+    superseded: bool | None = None
+
+    def has_superseded(self) -> bool:
+        if self.superseded is not None:
+            return self.superseded
+        sm = self.slot_mapping_np
+        return bool(sm.size and np.any((sm < 0) & (self.row_ctx_np > 0)))
+
     def to(self, device: torch.device) -> "StepMetadata":
         """Upload every array with one host-to-device copy (views into one buffer);
         the parts' arrays get copies of their own."""
@@ -228,6 +238,7 @@ class ColumnsRoute(NamedTuple):
     head_dim: int
     num_xcds: int
     num_cus: int
+    dtype: int = 2
 
 
 def _i32_columns(*columns):
@@ -238,7 +249,6 @@ def _i32_columns(*columns):
     return cols, [c.ctypes.data_as(ctypes.c_void_p) for c in cols]
 
 
-    dtype: int = 2
 def columns_partition(pos0s, new_rows, route: ColumnsRoute, other_partitions: int = 0) -> int:
     """tb_prefill_columns_partition: positions per partition of the step's column rows
     (``other_partitions``: those of its other rows)."""
@@ -421,6 +431,9 @@ def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, bl
             if column_seqs:
                 for s0, _, _, n in column_seqs:
                     tiled[s0:s0 + n] = True               # served by tb_paged_prefill_columns
+                part = columns_partition([x[2] for x in column_seqs], [x[3] for x in column_seqs], columns_route,
+                                         int(nparts_by_row[~tiled].sum()))
+                for s0, _, _, n in column_seqs:
                     nparts_by_row[s0:s0 + n] = (row_ctx_by_row[s0:s0 + n] + part - 1) // part
                 columns_work = build_columns_work(*zip(*column_seqs), part, columns_route)
         if tile_prefill:
@@ -431,9 +444,6 @@ def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, bl
                     tiled[s0:s0 + n] = True               # served by tiles, not work items
                     rc = row_ctx_by_row[s0:s0 + n]
                     nparts_by_row[s0:s0 + n] = (rc + TILE_PARTITION - 1) // TILE_PARTITION
-                part = columns_partition([x[2] for x in column_seqs], [x[3] for x in column_seqs], columns_route,
-                                         int(nparts_by_row[~tiled].sum()))
-                for s0, _, _, n in column_seqs:
                     for r in range(0, n, TILE_ROWS):
                         rows = min(TILE_ROWS, n - r)
                         pos0 = c - n + r
@@ -522,6 +532,7 @@ def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, bl
         prefill_max_tiles=prefill_tiles_max,
         columns_work_np=columns_work,
         num_columns_work=0 if columns_work is None else int(columns_work.shape[0]),
+        superseded=bool(np.any((slots < 0) & (row_ctx_by_row > 0))),
     )
 
 

@@ -151,8 +151,7 @@ def workspace_for(meta: StepMetadata, num_heads: int, head_dim: int,
     if meta.max_parts_per_row <= 1:
         return None
     need = int(_lib.lib().tb_paged_attention_workspace_bytes(meta.total_partitions, num_heads, head_dim))
-    key = (device.index if device.index is not None else torch.cuda.current_device(),
-           torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index if device.index is not None else torch.cuda.current_device(), _lib.stream_handle(device))
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < need:
         ws = torch.empty(max(need, 1 << 20), dtype=torch.uint8, device=device)
@@ -398,8 +397,7 @@ class DecodeBuffers:
 def decode_buffers(device: torch.device, piece_bytes: int, units: int) -> DecodeBuffers:
     """Cached per device and stream (calls on one stream are ordered; calls on two
     streams must not share counters); grown on demand, new counters zeroed."""
-    key = (device.index if device.index is not None else torch.cuda.current_device(),
-           torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index if device.index is not None else torch.cuda.current_device(), _lib.stream_handle(device))
     b = _DECODE_WORKSPACES.get(key)
     if b is None or b.pieces.numel() < piece_bytes or b.units < units:
         b = DecodeBuffers(device, max(piece_bytes, 0 if b is None else b.pieces.numel()),
@@ -506,8 +504,7 @@ def paged_attention(q: torch.Tensor, pool: torch.Tensor, meta: StepMetadata, *, 
         if fused:
             # a slot written by rows of both parts: each part's own slot mapping cannot
             # see it, the whole step's can (the superseded writer holds -1)
-            sm = meta.slot_mapping_np
-            if sm.size and np.any((sm < 0) & (meta.row_ctx_np > 0)):
+            if meta.has_superseded():
                 raise ValueError("two rows of the step write one pool slot; the fused append cannot serve "
                                  "the step: append with kv_append, then call paged_attention without k_new")
         for r0, r1, m in meta.parts:
@@ -559,8 +556,7 @@ def paged_attention(q: torch.Tensor, pool: torch.Tensor, meta: StepMetadata, *, 
         elif not meta.decode_only or meta.num_prefill_tiles or meta.num_prefill_work or meta.num_columns_work:
             raise ValueError("fused append needs a decode-only step (one query row per sequence) or a step of "
                              "whole prefills only")
-        sm = meta.slot_mapping_np
-        if sm.size and np.any((sm < 0) & (meta.row_ctx_np > 0)):
+        if meta.has_superseded():
             # a superseded writer of a shared slot: the kernel would store and read each
             # row's own K/V where the reference's last writer wins (kv_cache.py:33-38)
             raise ValueError("two decode rows write one pool slot; the fused append cannot serve the "
@@ -646,30 +642,54 @@ class BlockCopyPlan:
     live on the device, so ``launch`` makes no host round trip and can be
     captured in a HIP graph (the pools must stay allocated while it is in use)."""
 
-    def __init__(self, pools: list[torch.Tensor], src, dst):
+    def __init__(self, pools: list[torch.Tensor], src, dst, *, same_stream: bool = False):
         if not pools:
             raise ValueError("no layer pools")
-        nb = pools[0].shape[0]
-        for p in pools:
-            _check_pool(p)
-            if p.shape != pools[0].shape or p.dtype != pools[0].dtype or p.device != pools[0].device:
-                raise ValueError("all layer pools must share shape, dtype and device")
+        first = pools[0]
+        nb = _check_pool(first)[0]
+        shape, dtype, device, strides = first.shape, first.dtype, first.device, first.stride()
+        for p in pools[1:]:
+            if p.dtype != dtype or p.device != device or p.stride() != strides or p.shape != shape:
+                _check_pool(p)
+                if p.shape != shape or p.dtype != dtype or p.device != device:
+                    raise ValueError("all layer pools must share shape, dtype and device")
         s_np = np.asarray(src.cpu() if isinstance(src, torch.Tensor) else src, dtype=np.int64).reshape(-1)
         d_np = np.asarray(dst.cpu() if isinstance(dst, torch.Tensor) else dst, dtype=np.int64).reshape(-1)
-        if s_np.size != d_np.size:
+        n = int(s_np.size)
+        if n != d_np.size:
             raise ValueError("src and dst differ in length")
-        if d_np.size != np.unique(d_np).size:
+        ids = np.concatenate([s_np, d_np])
+        if n and (ids.min() < 0 or ids.max() >= nb):
+            if np.unique(d_np).size != n:
+                raise ValueError("dst block ids must be distinct")
+            if np.intersect1d(s_np, d_np).size:
+                raise ValueError("a dst block is also a src block; split the copy into rounds")
+            bad = "src" if s_np.min() < 0 or s_np.max() >= nb else "dst"
+            raise IndexError(f"{bad} holds a block id outside [0, {nb})")
+        is_dst = np.zeros(nb, dtype=bool)     # marks instead of sorts: a fifth of the time at 1024 pairs
+        is_dst[d_np] = True
+        if int(np.count_nonzero(is_dst)) != n:
             raise ValueError("dst block ids must be distinct")
-        if np.intersect1d(s_np, d_np).size:
+        if is_dst[s_np].any():
             raise ValueError("a dst block is also a src block; split the copy into rounds")
-        self.device = pools[0].device
+        self.device = device
         self.num_blocks = nb
         self.num_layers = len(pools)
-        self.num_pairs = int(s_np.size)
-        self.block_bytes = pools[0][0].numel() * pools[0].element_size()
-        self.src = _block_ids("src", s_np, nb, self.device)
-        self.dst = _block_ids("dst", d_np, nb, self.device)
-        self.ptrs = torch.tensor([p.data_ptr() for p in pools], dtype=torch.int64).to(self.device)
+        self.num_pairs = n
+        self.block_bytes = first[0].numel() * first.element_size()
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("a copy round's ids cannot be uploaded while a graph is being captured: build its "
+                               "BlockCopyPlan first")
+        # pool pointers (64-bit), then src and dst ids (32-bit): one pinned buffer, one copy; waited
+        # for unless the caller launches on this stream only (same_stream)
+        L = self.num_layers
+        host = torch.empty(2 * L + 2 * n, dtype=torch.int32, pin_memory=True)
+        flat = host.numpy()
+        flat[:2 * L].view(np.int64)[:] = [p.data_ptr() for p in pools]
+        flat[2 * L:] = ids
+        buf = host.to(device, non_blocking=same_stream)
+        self.ptrs = buf[:2 * L].view(torch.int64)
+        self.src, self.dst = buf[2 * L:2 * L + n], buf[2 * L + n:]
 
     def launch(self) -> None:
         st = _lib.lib().tb_block_copy(self.ptrs.data_ptr(), self.num_layers, self.num_blocks, self.src.data_ptr(),
@@ -682,7 +702,7 @@ def block_copy(pools: list[torch.Tensor], src, dst) -> None:
     """K3: pool_l[dst[i]] <- pool_l[src[i]] for every layer pool l, one launch."""
     if not pools:
         return
-    BlockCopyPlan(pools, src, dst).launch()
+    BlockCopyPlan(pools, src, dst, same_stream=True).launch()
 
 
 def block_gather(pool: torch.Tensor, blocks, staging: torch.Tensor) -> None:
