@@ -64,8 +64,9 @@ def test_more_chunks_than_one_read_of_block_ids(BS):
 def test_rows_of_one_and_two_partitions_in_one_tile(dtype):
     """Rows that cross the first partition's end inside a tile of 18 rows: the second
     partition's workgroup leaves the earlier rows alone."""
-    meta = check(case(9, 14, 2, 64, 16, dtype, [1000], [0]))
-    assert 0 < meta.num_split_rows < 1000
+    c = case(9, 14, 2, 64, 16, dtype, [2500], [0])
+    meta = check(c)
+    assert 0 < meta.num_split_rows < 2500
 
 
 def test_whole_rows_when_the_step_fills_the_gpu():

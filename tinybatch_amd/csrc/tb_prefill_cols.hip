@@ -118,15 +118,19 @@ struct cshape {
   }
 };
 
-template <typename Tag, int D>
-__global__ __launch_bounds__(64 * cshape<D>::NW, 2) void paged_prefill_columns_kernel(const cols_args a) {
+// SP = 2: two sets of NW waves on the same columns, set sp taking chunks sp, sp + 2, ... of
+// the range through a ring of its own; their states merge in LDS at the end.
+template <typename Tag, int D, int SP>
+__global__ __launch_bounds__(64 * cshape<D>::NW * SP, 2) void paged_prefill_columns_kernel(const cols_args a) {
   using S = cshape<D>;
   using M = cmath<Tag>;
   typedef typename smath<Tag>::scalar_t scalar_t;
   constexpr int RB = S::RB, TB = S::TB, CK = S::CK, KS = S::KS, NB = S::NB;
-  __shared__ __align__(1024) char lds[S::RING * S::SLOT];
+  __shared__ __align__(1024) char lds_all[SP * S::RING * S::SLOT];
 
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wave_id = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wave = wave_id % S::NW, sp = wave_id / S::NW;   // the wave's columns, its set of chunks
+  char* const lds = lds_all + sp * (S::RING * S::SLOT);
   const int lane = threadIdx.x & 63, lcol = lane & 31, half = lane >> 5;
   const int4 w0 = a.work[2 * blockIdx.x], w1 = a.work[2 * blockIdx.x + 1];
   const int row0 = w0.x, seq = w0.y, pos0 = w0.z, nrows = w0.w;
@@ -168,7 +172,7 @@ __global__ __launch_bounds__(64 * cshape<D>::NW, 2) void paged_prefill_columns_k
   const int lt = wave;                          // the tile of a chunk this wave loads, K and V
   const int lrow = lane / S::VCOLS, lpiece = lane % S::VCOLS;
   // lane j: the block of this wave's tile in chunk id0 + j
-  int id0 = c_begin;
+  int id0 = c_begin + sp;
   auto load_ids = [&](int c) {
     const int t = min(4 * (c + lane) + lt, last_tile);
     int b = table[(t << 4) >> a.log2_bs];
@@ -194,7 +198,7 @@ __global__ __launch_bounds__(64 * cshape<D>::NW, 2) void paged_prefill_columns_k
     }
   };
   asm volatile("" : "+v"(ids));                 // the block ids have landed: no wait inside the loop
-  if (c_begin < c_end) issue(c_begin, 0);
+  if (c_begin + sp < c_end) issue(c_begin + sp, 0);
 
   // ---- q rotated (RoPE at the column's position), complete here ----
   if (a.rope.cos) {
@@ -329,20 +333,45 @@ __global__ __launch_bounds__(64 * cshape<D>::NW, 2) void paged_prefill_columns_k
     }
   };
 
-  // Chunk k of the range (relative to c_begin) lies in ring slot k % RING.
-  const int n = c_end - c_begin;
-  const int n_wave = wave_busy ? min(c_end - 1, wave_last / CK) - c_begin + 1 : 0;   // this wave's chunks
+  // The set's chunk k, c_begin + SP k + sp, lies in slot k % RING of its ring.
+  const int n = (c_end - c_begin + SP - 1) / SP;
+  const int c_wave = wave_busy ? min(c_end - 1, wave_last / CK) : -1;   // this wave's last chunk
   for (int k = 0; k < n; ++k) {
     // the wave's loads of chunk k have landed and its LDS reads of chunk k - 1 are done:
     // behind the barrier all of chunk k is in LDS and the slot of chunk k - 1 is free
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (k + 1 < n) issue(c_begin + k + 1, (k + 1) % S::RING);
-    if (k < n_wave) {
+    const int c = c_begin + SP * k + sp;
+    if (c + SP < c_end) issue(c + SP, (k + 1) % S::RING);
+    if (c <= c_wave) {
       const int slot = k % S::RING;
       scores(slot);
-      softmax(c_begin + k);
+      softmax(c);
       values(slot);
     }
+  }
+
+  if constexpr (SP == 2) {                      // set 1's state to set 0 (log-sum-exp)
+    float* const slot = reinterpret_cast<float*>(lds_all) + wave * (64 * (16 * NB + 2)) + lane;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // every read of the chunks is done
+    if (sp == 1) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) slot[64 * (16 * b + r)] = acc[b][r];
+      slot[64 * 16 * NB] = m;
+      slot[64 * (16 * NB + 1)] = l;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (sp == 1) return;
+    const float m1 = slot[64 * 16 * NB], l1 = slot[64 * (16 * NB + 1)];
+    const float m_new = fmaxf(m, m1), m_safe = m_new == -INFINITY ? 0.f : m_new;
+    const float f0 = fast_exp2(m - m_safe), f1 = fast_exp2(m1 - m_safe);   // 0 for a set that saw nothing
+    m = m_new;
+    l = l * f0 + l1 * f1;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[b][r] = acc[b][r] * f0 + slot[64 * (16 * b + r)] * f1;
   }
 
   l = sum_xor32(l);
@@ -589,6 +618,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void paged_prefill_columns_f3
 namespace {
 
 constexpr int COLS = tb::cshape<64>::COLS, CHUNK = tb::cshape<64>::CK;
+constexpr int COLS_SHARED = 256;   // workgroups up to which two sets of waves share one's chunks
 static_assert(COLS == tb::cshape<128>::COLS && CHUNK == tb::cshape<128>::CK, "one work list for both head dims");
 
 struct col_entry {
@@ -639,7 +669,14 @@ extern "C" int32_t tb_prefill_columns_partition(const int32_t* pos0, const int32
   const bool d64 = head_dim == 64, f32 = dtype == TB_DTYPE_F32;
   const double alone = f32 ? (d64 ? 4.0 : 8.0) : d64 ? 1.0 : 1.6, full = f32 ? (d64 ? 3.6 : 7.2) : d64 ? 0.65 : 1.05;
   const double share = full * (double)total / num_cus;
-  auto span = [&](int chunks) { return std::max(alone * chunks, share + 0.5 * full * chunks); };
+  auto span = [&](int chunks) {
+    int64_t wgs = 0;
+    for (int i = 0; i < num_seqs; ++i)
+      for (int c = 0; c < new_rows[i] * rep; c += COLS)
+        wgs += ((columns_limit(pos0[i], new_rows[i], rep, c) + CHUNK - 1) / CHUNK + chunks - 1) / chunks * num_kv_heads;
+    const double one = !f32 && wgs <= COLS_SHARED ? 0.66 * alone : alone;   // two sets of waves on its chunks
+    return std::max(one * chunks, share + 0.5 * full * chunks);
+  };
   int best = longest + 1;                              // longer than every context: no row is split
   double cost = span(longest);
   for (int part = 4; part < longest; part += part < 16 ? 2 : part < 64 ? 8 : 32) {
@@ -688,12 +725,15 @@ extern "C" int32_t tb_build_prefill_columns_work(const int32_t* first_row, const
         }
       }
   // Entry g runs on XCD g % num_xcds: the entries in (kv head, sequence) order are cut into
-  // runs of equal work, one per XCD, so that few K/V ranges pass through each L2.
+  // runs of equal work, one per XCD, so that few K/V ranges pass through each L2; up to one
+  // entry per CU, into runs of equal length (every entry then has a CU).
+  const bool one_each = (int64_t)entries.size() <= num_cus;
+  if (one_each) total = (int64_t)entries.size();
   const int X = num_xcds, per = std::max(1, num_cus / X);
   std::vector<std::vector<col_entry>> bins(X);
   int64_t at = 0;
   for (const col_entry& e : entries) {
-    const int64_t w = e.chunks + 2;
+    const int64_t w = one_each ? 1 : e.chunks + 2;
     bins[std::min<int64_t>(X - 1, (2 * at + w) * X / (2 * total))].push_back(e);
     at += w;
   }
@@ -729,6 +769,24 @@ extern "C" int32_t tb_build_prefill_columns_work(const int32_t* first_row, const
     }
   return TB_OK;
 }
+
+namespace {
+
+// At most one workgroup per CU (256): two sets of waves share its chunks, which then take
+// 0.66 us each instead of 1.0 (head dim 64). Twelve prefix hits of 40..400 rows after
+// 600..3600 positions, 4 fp16 layers with the append: 149 us unsplit against 162 for one set
+// of waves and rows split at 896 positions. Past 256 workgroups one set each leaves room
+// for a second workgroup on the CU, whose start and end then overlap.
+template <typename Tag, int D>
+void launch_columns(const tb::cols_args& a, int num_work, hipStream_t stream) {
+  constexpr int T = 64 * tb::cshape<D>::NW;
+  if (num_work <= COLS_SHARED)
+    hipLaunchKernelGGL((tb::paged_prefill_columns_kernel<Tag, D, 2>), dim3(num_work), dim3(2 * T), 0, stream, a);
+  else
+    hipLaunchKernelGGL((tb::paged_prefill_columns_kernel<Tag, D, 1>), dim3(num_work), dim3(T), 0, stream, a);
+}
+
+}  // namespace
 
 extern "C" int32_t tb_paged_prefill_columns(const void* q, int64_t q_row_stride, const void* pool, int64_t num_blocks,
                                             void* out, int64_t out_row_stride, const int32_t* block_tables,
@@ -788,17 +846,15 @@ extern "C" int32_t tb_paged_prefill_columns(const void* q, int64_t q_row_stride,
   while ((1 << a.log2_bs) < block_size) ++a.log2_bs;
   a.scale_log2e = scale * 1.4426950408889634f;
   a.rope = rope_tables{rope_cos, rope_sin, rope_max_position};
-  const dim3 grid(num_work), block(64 * cshape<64>::NW);
   const bool d64 = head_dim == 64;
   if (dtype == TB_DTYPE_F32) {
+    const dim3 grid(num_work), block(256);
     if (d64) hipLaunchKernelGGL((paged_prefill_columns_f32_kernel<64>), grid, block, 2 * fshape<64>::SLOT, stream, a);
     else hipLaunchKernelGGL((paged_prefill_columns_f32_kernel<128>), grid, block, 2 * fshape<128>::SLOT, stream, a);
   } else if (dtype == TB_DTYPE_F16) {
-    if (d64) hipLaunchKernelGGL((paged_prefill_columns_kernel<f16_t, 64>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((paged_prefill_columns_kernel<f16_t, 128>), grid, block, 0, stream, a);
+    d64 ? launch_columns<f16_t, 64>(a, num_work, stream) : launch_columns<f16_t, 128>(a, num_work, stream);
   } else {
-    if (d64) hipLaunchKernelGGL((paged_prefill_columns_kernel<bf16_t, 64>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((paged_prefill_columns_kernel<bf16_t, 128>), grid, block, 0, stream, a);
+    d64 ? launch_columns<bf16_t, 64>(a, num_work, stream) : launch_columns<bf16_t, 128>(a, num_work, stream);
   }
   if (num_split_rows > 0)
     combine_split_rows(dtype, head_dim, num_heads, out, out_row_stride * eb, split_rows, num_split_rows, a.ws_acc, a.ws_ml,
