@@ -111,7 +111,7 @@ struct attn_args {
 //   O^T[d][head]   += V^T[d][pos] . P^T[pos][head]  A: V[pos 4 lg + j][4 lc + i], B: the S^T registers
 // (k index lg of a product stands for dim 16 c + 4 lg + i, or position 4 lg + j, in both
 // operands, so every operand is a whole 16-byte load used component by component). A
-// score's dims are summed in chains of 8. The waves' states merge in LDS.
+// score's dims are summed in chains of 4. The waves' states merge in LDS.
 //
 // Bound by latency: at 8 rows of up to 250 positions a call is one chain of table read, K/V
 // read, 32 products a wave and the merge on 16 CUs. us per layer in a
@@ -215,24 +215,21 @@ __global__ __launch_bounds__(64 * NW_) void paged_attn_f32_kernel(const attn_arg
           for (int c = 0; c < VC; ++c) st16_through(vslot + j * RB + 16 * lc + 256 * c, v[j][c]);
         }
     }
-    float4_t sh[2];                        // chains of 8 dims, added pairwise
+    float4_t sh[4];                        // chains of 4 dims, added pairwise
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int i = 0; i < 4; ++i) {
       float4_t sc[KC];
 #pragma unroll
-      for (int c = 0; c < KC; ++c) {
-        sc[c] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 2 * h; i < 2 * h + 2; ++i)
-          sc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(bits_to_f32(k[c].w[i]), bits_to_f32(q[c].w[i]), sc[c], 0, 0, 0);
-      }
+      for (int c = 0; c < KC; ++c)
+        sc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(bits_to_f32(k[c].w[i]), bits_to_f32(q[c].w[i]),
+                                                     float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
       for (int st = 1; st < KC; st *= 2)
 #pragma unroll
         for (int c = 0; c < KC; c += 2 * st) sc[c] += sc[c + st];
-      sh[h] = sc[0];
+      sh[i] = sc[0];
     }
-    float4_t s = sh[0] + sh[1];            // positions t0 + 4 lg + j of head lc
+    float4_t s = (sh[0] + sh[1]) + (sh[2] + sh[3]);    // positions t0 + 4 lg + j of head lc
 #pragma unroll
     for (int j = 0; j < 4; ++j) s[j] = vpos + j < p1 ? s[j] * a.scale_log2e : -INFINITY;
     const float cm = max_xor32(max_xor16(max_f32(max_f32(s[0], s[1]), max_f32(s[2], s[3]))));

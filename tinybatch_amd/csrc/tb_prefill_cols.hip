@@ -410,13 +410,13 @@ __global__ __launch_bounds__(64 * cshape<D>::NW * SP, 2) void paged_prefill_colu
 // 32 positions. k index half of a product stands for dim 8 c + 4 half + i of the K rows and
 // q (whole 16-byte loads, component by component), and for position 8 (r / 4) + 4 half +
 // r % 4 of V and P, whose B operand is then register r of the scores as it is. A
-// score's dims are summed in eight chains, and a chunk's P.V apart from the chunks before
-// it, so that rounding stays at the level of the row-by-row kernel's (distance from 64-bit
-// results 1.4e-7; 2.2e-7 with two chains and one running sum).
+// score's dims are summed in 16 chains, and a chunk's P.V in two, apart from the chunks
+// before it, so that rounding stays below the row-by-row kernel's (distance from 64-bit
+// results 1.30e-7 against 1.45e-7; 2.2e-7 with two chains and one running sum).
 //
 // Bound by the fp32 matrix rate (154 TFLOP/s for a library product here). us per
-// layer for six prompts of 201..687 tokens at 14 / 2 heads of 64: 59 with the append, against
-// 119 for one work item per row.
+// layer for six prompts of 201..687 tokens at 14 / 2 heads of 64: 47 to 50 with the append,
+// against 119 for one work item per row.
 template <int D>
 struct fshape {
   static constexpr int RB = 4 * D;
@@ -527,16 +527,16 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void paged_prefill_columns_f3
     if (k >= n_wave) continue;
     const int c = c_begin + k;
     const char* const base = flds + (k & 1) * S::SLOT;
-    float16_t sh[2];                            // chains of 8 dims (D / 8 at head dim 128), added pairwise
+    float16_t sh[4];                            // chains of D / 16 dims, added pairwise
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < 4; ++h) {
       float16_t d4[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) d4[i][r] = 0.f;
 #pragma unroll
-      for (int cc = h * KC / 2; cc < (h + 1) * KC / 2; ++cc) {
+      for (int cc = h * KC / 4; cc < (h + 1) * KC / 4; ++cc) {
         const vec16 kv = ld16(base + lcol * RB + 16 * ((2 * cc + half) ^ S::kswz(lcol)));
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -544,7 +544,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void paged_prefill_columns_f3
       }
       sh[h] = (d4[0] + d4[1]) + (d4[2] + d4[3]);
     }
-    float16_t sc = sh[0] + sh[1];
+    float16_t sc = (sh[0] + sh[1]) + (sh[2] + sh[3]);
     if (CK * c + CK - 1 > wave_first) {         // the chunk crosses the diagonal of some column
       asm volatile("");
 #pragma unroll
@@ -569,19 +569,18 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void paged_prefill_columns_f3
     l += (((sc[0] + sc[1]) + (sc[2] + sc[3])) + ((sc[4] + sc[5]) + (sc[6] + sc[7]))) +
          (((sc[8] + sc[9]) + (sc[10] + sc[11])) + ((sc[12] + sc[13]) + (sc[14] + sc[15])));
     const char* const vb = base + S::HALF + 4 * half * RB + 4 * lcol;
-    float16_t pv[NB];                           // the chunk's own sum: shorter chains than one over all positions
+    // the chunk's own sums, in two chains: shorter than one over all positions
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
+    for (int b = 0; b < NB; ++b) {
+      float16_t pv[2];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) pv[b][r] = 0.f;
+      for (int r = 0; r < 16; ++r) pv[0][r] = pv[1][r] = 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-        pv[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-            *reinterpret_cast<const float*>(vb + (8 * (r >> 2) + (r & 3)) * RB + 128 * b), sc[r], pv[b], 0, 0, 0);
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] += pv[b];
+      for (int r = 0; r < 16; ++r)
+        pv[r & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+            *reinterpret_cast<const float*>(vb + (8 * (r >> 2) + (r & 3)) * RB + 128 * b), sc[r], pv[r & 1], 0, 0, 0);
+      acc[b] += pv[0] + pv[1];
+    }
   }
 
   l = sum_xor32(l);

@@ -241,12 +241,11 @@ class ColumnsRoute(NamedTuple):
     dtype: int = 2
 
 
-def _i32_columns(*columns):
-    """The columns as int32 arrays and their pointers."""
-    import ctypes
-
-    cols = [np.ascontiguousarray(np.asarray(x, dtype=np.int32).reshape(-1)) for x in columns]
-    return cols, [c.ctypes.data_as(ctypes.c_void_p) for c in cols]
+def _column_arrays(first_rows, seqs, pos0s, new_rows) -> tuple[np.ndarray, list[int]]:
+    """The four per-sequence columns as rows of one int32 array, and the rows' addresses."""
+    a = np.array([first_rows, seqs, pos0s, new_rows], dtype=np.int32).reshape(4, -1)
+    at = a.__array_interface__["data"][0]
+    return a, [at + 4 * a.shape[1] * i for i in range(4)]
 
 
 def columns_partition(pos0s, new_rows, route: ColumnsRoute, other_partitions: int = 0) -> int:
@@ -254,10 +253,9 @@ def columns_partition(pos0s, new_rows, route: ColumnsRoute, other_partitions: in
     (``other_partitions``: those of its other rows)."""
     from . import _lib
 
-    cols, ptrs = _i32_columns(pos0s, new_rows)
-    p = int(_lib.lib().tb_prefill_columns_partition(*ptrs, cols[0].size, route.num_heads, route.num_kv_heads,
-                                                    route.head_dim, route.dtype, route.num_cus,
-                                                    other_partitions))
+    a, ptrs = _column_arrays(pos0s, pos0s, pos0s, new_rows)
+    p = int(_lib.lib().tb_prefill_columns_partition(ptrs[2], ptrs[3], a.shape[1], route.num_heads, route.num_kv_heads,
+                                                    route.head_dim, route.dtype, route.num_cus, other_partitions))
     if p < 0:
         _lib.check(p, "tb_prefill_columns_partition")
     return p
@@ -269,13 +267,19 @@ def build_columns_work(first_rows, seqs, pos0s, new_rows, partition: int, route:
 
     from . import _lib
 
-    cols, ptrs = _i32_columns(first_rows, seqs, pos0s, new_rows)
-    args = (*ptrs, cols[0].size, route.num_heads, route.num_kv_heads, partition, route.num_xcds, route.num_cus)
+    a, ptrs = _column_arrays(first_rows, list(seqs), pos0s, new_rows)
+    args = (*ptrs, a.shape[1], route.num_heads, route.num_kv_heads, partition, route.num_xcds, route.num_cus)
     lib, n = _lib.lib(), ctypes.c_int32()
-    _lib.check(lib.tb_build_prefill_columns_work(*args, None, 0, ctypes.byref(n)), "tb_build_prefill_columns_work")
-    work = np.zeros((max(n.value, 1), 8), dtype=np.int32)
-    _lib.check(lib.tb_build_prefill_columns_work(*args, work.ctypes.data_as(ctypes.c_void_p), n.value, ctypes.byref(n)),
-               "tb_build_prefill_columns_work")
+    # room for the entries (128 columns each) and as many padding ones; the exact count if that is short
+    rep = route.num_heads // route.num_kv_heads
+    room = sum((int(r) * rep // 128 + 1) * ((int(p) + int(r)) // partition + 1) for p, r in zip(pos0s, new_rows))
+    room = 2 * room * route.num_kv_heads + 8 * route.num_xcds
+    work = np.empty((room, 8), dtype=np.int32)
+    st = lib.tb_build_prefill_columns_work(*args, work.__array_interface__["data"][0], room, ctypes.byref(n))
+    if st != _lib.TB_OK and n.value > room:
+        work = np.empty((n.value, 8), dtype=np.int32)
+        st = lib.tb_build_prefill_columns_work(*args, work.__array_interface__["data"][0], n.value, ctypes.byref(n))
+    _lib.check(st, "tb_build_prefill_columns_work")
     return work[:n.value]
 
 
