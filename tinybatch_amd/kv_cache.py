@@ -71,7 +71,9 @@ class PagedKVCache:
         attention() / decode_step() with this metadata then run that kernel; a
         prefill-only step goes to tb_paged_prefill, and a step of whole prefills
         beside a run of decode rows to tb_paged_prefill and the decode kernel, each
-        on its own rows (ops.attach_split_parts), when the decode rows gain by it.
+        on its own rows (ops.attach_split_parts), when the decode rows gain by it. In any
+        other step (longer contexts, fp32) sequences of >= 16 new rows go to
+        tb_paged_prefill_columns (ops.columns_route).
         """
         pos_key = (positions, positions._version) if isinstance(positions, torch.Tensor) else list(positions)
         for e in self._meta_cache:
@@ -84,8 +86,8 @@ class PagedKVCache:
                 return e["meta"]
         # 16-bit pools serve long runs of new rows (prefills) with the tile kernel; a
         # step of prefills only (every sequence >= 16 new rows, its context within
-        # the kernel's limit) goes to tb_paged_prefill instead: a step that also has
-        # decode rows keeps them in the one launch with the tiles
+        # the kernel's limit) goes to tb_paged_prefill instead; in other steps such runs go
+        # to the column tiles, decode rows and short tails to the work items beside them
         tile = self.pools[0].dtype in (torch.float16, torch.bfloat16)
         route = None
         if num_heads is not None and context_lens is not None and self.device.type == "cuda" and tile:
