@@ -11,6 +11,7 @@ import pytest
 import torch
 
 from oracle import reference_path as ref
+from test_prefill_columns_work import both_routes
 from test_prefill_stream_gpu import DEV, TOL, case
 from tinybatch_amd import layer_ops, ops
 from tinybatch_amd.metadata import TILE_PARTITION, build_step_metadata
@@ -108,3 +109,14 @@ def test_rope_equals_rotating_first(dtype):
     got = ops.paged_attention(q, pool, meta, num_heads=14, rope=ops.Rope(cos, sin))
     want = ops.paged_attention(rotated, pool, meta, num_heads=14)
     assert torch.equal(got, want)
+
+
+def test_fused_append_refused_beside_column_rows():
+    """tb_paged_prefill would append its own rows and the column tiles read unwritten ones."""
+    meta = both_routes().to(DEV)
+    pool = torch.zeros(70, 2, 2, 16, 64, dtype=torch.bfloat16, device=DEV)
+    q = torch.zeros(1100, 14, 64, dtype=torch.bfloat16, device=DEV)
+    kv = torch.ones(1100, 2, 64, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(ValueError, match="fused append"):
+        ops.paged_attention(q, pool, meta, num_heads=14, k_new=kv, v_new=kv)
+    assert not pool.any()

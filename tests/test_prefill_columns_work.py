@@ -5,8 +5,9 @@ scratch than the tiles did, past the static scratch."""
 import numpy as np
 import pytest
 
-from tinybatch_amd.metadata import (TILE_PARTITION, ColumnsRoute, build_columns_work, build_step_metadata,
-                                    columns_partition)
+from tinybatch_amd.kv_cache import PagedKVCache
+from tinybatch_amd.metadata import (TILE_PARTITION, ColumnsRoute, PrefillRoute, build_columns_work,
+                                    build_step_metadata, columns_partition)
 
 
 def covered(first, pos0, rows, hq, hkv, work, part):
@@ -61,3 +62,20 @@ def test_metadata_counts_partitions_of_the_columns():
     assert m.num_columns_work and m.num_prefill_tiles == 0 and m.num_work_items == 1
     assert np.diff(m.row_part_off_np).tolist() == [-(-(2001 + i) // part) for i in range(40)] + [1]
     assert m.split_rows_np[:, 0].tolist() == list(range(40))
+
+
+def both_routes():
+    """A 100-row prompt for tb_paged_prefill beside a 1000-row one for the column tiles."""
+    return build_step_metadata(list(range(100)) + list(range(1000)), [(0, 100), (100, 1100)],
+                               [list(range(7)), list(range(7, 70))], [100, 1000], block_size=16, num_blocks=70,
+                               partition_tokens=256, rows_per_item=2, tile_prefill=True,
+                               prefill_route=PrefillRoute(2, 64, 560, 8), columns_route=ColumnsRoute(14, 2, 64, 8, 256))
+
+
+def test_column_rows_are_not_appended_by_the_attention():
+    m = both_routes()
+    assert m.num_prefill_work and m.num_columns_work and not m.num_work_items and not m.num_prefill_tiles
+    assert not PagedKVCache._fusable(m) and not m.whole_prefills_only()
+    only = build_step_metadata(list(range(100)), [(0, 100)], [list(range(7))], [100], block_size=16, num_blocks=7,
+                               partition_tokens=256, prefill_route=PrefillRoute(2, 64, 560, 8))
+    assert only.whole_prefills_only() and PagedKVCache._fusable(only)

@@ -205,7 +205,7 @@ class PagedKVCache:
             return False                                  # a superseded writer: the separate append
         if meta.parts is not None or meta.decode_only:
             return True
-        return bool(meta.num_prefill_work and not meta.num_work_items and not meta.num_prefill_tiles)
+        return meta.whole_prefills_only()
 
     def decode_step(self, layer: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, meta: StepMetadata,
                     *, num_heads: int | None = None, scale: float | None = None,

@@ -125,6 +125,12 @@ class StepMetadata:
         sm = self.slot_mapping_np
         return bool(sm.size and np.any((sm < 0) & (self.row_ctx_np > 0)))
 
+    def whole_prefills_only(self) -> bool:
+        """Every row is a tb_paged_prefill row, which that kernel can append itself: no work
+        items or tiles, and no column rows (their new K/V must be in the pool first)."""
+        return bool(self.num_prefill_work and not self.num_work_items and not self.num_prefill_tiles
+                    and not self.num_columns_work)
+
     def to(self, device: torch.device) -> "StepMetadata":
         """Upload every array with one host-to-device copy (views into one buffer);
         the parts' arrays get copies of their own."""

@@ -549,7 +549,7 @@ def paged_attention(q: torch.Tensor, pool: torch.Tensor, meta: StepMetadata, *, 
     if k_new is not None or v_new is not None:
         if k_new is None or v_new is None:
             raise ValueError("k_new and v_new go together")
-        if meta.num_prefill_work and not meta.num_work_items and not meta.num_prefill_tiles:
+        if meta.whole_prefills_only():
             # whole prefill sequences only: tb_paged_prefill reads their new rows from
             # k_new / v_new (K rotated in the kernel with ``rope``) and stores them
             prefill_fused = True
