@@ -255,7 +255,8 @@ int32_t tb_paged_prefill(const void* q, int64_t q_row_stride, void* pool, int64_
  * The rows it serves must not also be given to tb_paged_attention as work items or tiles.
  * The K/V of the step's new rows must already be in the pool (append first).
  *   work: tb_build_prefill_columns_work's list (device memory, 16-byte aligned), num_work
- *     entries of 8 int32; row_part_offsets [num_rows + 1]: as tb_paged_attention takes it,
+ *     entries of 8 int32, built for this call's num_heads and num_kv_heads (its columns are
+ *     row * num_heads / num_kv_heads + head); row_part_offsets [num_rows + 1]: as tb_paged_attention takes it,
  *     with ceil(row_ctx / partition_tokens) partitions for every row served here;
  *   split_rows [num_split_rows][4] (row, first partial slot, count, 0): the rows whose
  *     partials this call merges at its end; 0 leaves them to a tb_paged_attention call that

@@ -20,12 +20,12 @@ from tinybatch_amd.model import rope_tables
 pytestmark = pytest.mark.gpu
 
 
-def metadata(c):
+def metadata(c, rows=None):
     dt, Hq, Hkv, D = c["dtype"], c["Hq"], c["Hkv"], c["D"]
     route = ops.columns_route(dt, Hq, Hkv, D, c["BS"], DEV)
     return build_step_metadata(c["pos"], c["slices"], c["tables"], c["ctx"], block_size=c["BS"], num_blocks=c["NB"],
                                partition_tokens=ops.partition_tokens(dt, D),
-                               rows_per_item=ops.rows_per_item(dt, Hq, Hkv), tile_prefill=True,
+                               rows_per_item=rows or ops.rows_per_item(dt, Hq, Hkv), tile_prefill=True,
                                columns_route=route).to(DEV)
 
 
@@ -120,3 +120,21 @@ def test_fused_append_refused_beside_column_rows():
     with pytest.raises(ValueError, match="fused append"):
         ops.paged_attention(q, pool, meta, num_heads=14, k_new=kv, v_new=kv)
     assert not pool.any()
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(28, 2), (4, 4), (2, 1)])
+def test_metadata_of_other_heads(Hq, Hkv, monkeypatch):
+    """Metadata built for 14 / 2 heads serves a call with other heads: a list of its own,
+    uploaded on the first call and not while a graph is captured."""
+    c = case(10, Hq, Hkv, 64, 16, torch.bfloat16, [100, 20], [900, 0])
+    want = ref.attention(c["q"], c["pool"], c["slices"], c["tables"], c["ctx"], Hq, Hkv)
+    meta = metadata({**c, "Hq": 14, "Hkv": 2}, rows=1)
+    q, pool = c["q"].to(DEV), c["pool"].to(DEV)
+    out = torch.full((120, Hq * 64), float("nan"), dtype=torch.bfloat16, device=DEV)
+    with monkeypatch.context() as m, pytest.raises(RuntimeError, match="call once"):
+        m.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+        ops.paged_attention(q, pool, meta, num_heads=Hq, out=out)
+    for _ in range(2):
+        got = ops.paged_attention(q, pool, meta, num_heads=Hq, out=out).cpu()
+        torch.testing.assert_close(got.float(), want.float(), **TOL)
+    assert len(meta.columns_other) == 1

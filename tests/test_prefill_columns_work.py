@@ -79,3 +79,13 @@ def test_column_rows_are_not_appended_by_the_attention():
     only = build_step_metadata(list(range(100)), [(0, 100)], [list(range(7))], [100], block_size=16, num_blocks=7,
                                partition_tokens=256, prefill_route=PrefillRoute(2, 64, 560, 8))
     assert only.whole_prefills_only() and PagedKVCache._fusable(only)
+
+
+@pytest.mark.parametrize("hq,hkv", [(14, 2), (28, 2), (7, 1), (4, 4), (32, 8)])
+def test_other_heads_get_a_list_of_their_own(hq, hkv):
+    """Metadata built for 14 / 2 heads, used with others: every (row, head) of the call once."""
+    m = build_step_metadata(list(range(900, 1000)), [(0, 100)], [list(range(63))], [1000], block_size=16, num_blocks=63,
+                            partition_tokens=256, columns_route=ColumnsRoute(14, 2, 64, 8, 256))
+    work = m.columns_list(hq, hkv)
+    assert (work is m.columns_work_np) == ((hq, hkv) == (14, 2))
+    covered([0], [900], [100], hq, hkv, work, m.columns_partition)

@@ -38,7 +38,7 @@ IndexError (kv_cache.py:35), a block id outside the pool raises IndexError
 from __future__ import annotations
 
 import itertools
-from dataclasses import dataclass
+from dataclasses import dataclass, field
 
 from typing import NamedTuple
 
@@ -106,10 +106,16 @@ class StepMetadata:
     prefill_max_tiles: int = 0
     prefill_work: torch.Tensor | None = None
     # prefill sequences of any context served by tb_paged_prefill_columns
-    # (build_step_metadata's columns_route): its work list [n, 8] and partition length
+    # (build_step_metadata's columns_route): its work list [n, 8], which holds for the heads
+    # of the route alone (columns_for lists other heads' columns), the sequences (first row,
+    # sequence, first position, new rows) and the partition length
     columns_work_np: np.ndarray | None = None
     num_columns_work: int = 0
     columns_work: torch.Tensor | None = None
+    columns_route: "ColumnsRoute | None" = None
+    columns_seqs: list | None = None
+    columns_partition: int = 0
+    columns_other: dict = field(default_factory=dict)
     # a mixed step served as sub-steps (split_step_parts): (first row, end row, the
     # sub-step's metadata with rows counted from the first row); the arrays above
     # still describe the whole step (its slot mapping serves the append)
@@ -130,6 +136,30 @@ class StepMetadata:
         items or tiles, and no column rows (their new K/V must be in the pool first)."""
         return bool(self.num_prefill_work and not self.num_work_items and not self.num_prefill_tiles
                     and not self.num_columns_work)
+
+    def columns_list(self, num_heads: int, num_kv_heads: int) -> np.ndarray:
+        """The column work list for these heads: columns_work_np for the route's own."""
+        r = self.columns_route
+        if r is None or (r.num_heads, r.num_kv_heads) == (num_heads, num_kv_heads):
+            return self.columns_work_np
+        return build_columns_work(*zip(*self.columns_seqs), self.columns_partition,
+                                  r._replace(num_heads=num_heads, num_kv_heads=num_kv_heads))
+
+    def columns_for(self, num_heads: int, num_kv_heads: int, device: torch.device) -> tuple[torch.Tensor, int]:
+        """The uploaded column work list for a call's heads, and its entries. A call with other
+        heads than the route's uploads a list of its own once (not while a graph is captured)."""
+        r = self.columns_route
+        if r is None or (r.num_heads, r.num_kv_heads) == (num_heads, num_kv_heads):
+            return self.columns_work, self.num_columns_work
+        key = (num_heads, num_kv_heads, device)
+        if key not in self.columns_other:
+            if torch.cuda.is_current_stream_capturing():
+                raise RuntimeError(f"metadata built for {r.num_heads} / {r.num_kv_heads} heads: a list for {num_heads} "
+                                   f"/ {num_kv_heads} cannot be uploaded while a graph is being captured; call once "
+                                   "before")
+            self.columns_other[key] = torch.from_numpy(self.columns_list(num_heads, num_kv_heads)).to(device)
+        work = self.columns_other[key]
+        return work, int(work.shape[0])
 
     def to(self, device: torch.device) -> "StepMetadata":
         """Upload every array with one host-to-device copy (views into one buffer);
@@ -407,7 +437,7 @@ def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, bl
     tiles: list[tuple[int, int, int, int, int]] = []
     stream_seqs: list[tuple[int, int, int, int]] = []
     column_seqs: list[tuple[int, int, int, int]] = []
-    columns_work = None
+    columns_work, columns_part = None, 0
     tiled = np.zeros(T, dtype=bool)
     nparts_by_row = np.zeros(T, dtype=np.int64)
     if tot and context_lens is not None:
@@ -441,11 +471,11 @@ def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, bl
             if column_seqs:
                 for s0, _, _, n in column_seqs:
                     tiled[s0:s0 + n] = True               # served by tb_paged_prefill_columns
-                part = columns_partition([x[2] for x in column_seqs], [x[3] for x in column_seqs], columns_route,
-                                         int(nparts_by_row[~tiled].sum()))
+                columns_part = columns_partition([x[2] for x in column_seqs], [x[3] for x in column_seqs],
+                                                 columns_route, int(nparts_by_row[~tiled].sum()))
                 for s0, _, _, n in column_seqs:
-                    nparts_by_row[s0:s0 + n] = (row_ctx_by_row[s0:s0 + n] + part - 1) // part
-                columns_work = build_columns_work(*zip(*column_seqs), part, columns_route)
+                    nparts_by_row[s0:s0 + n] = (row_ctx_by_row[s0:s0 + n] + columns_part - 1) // columns_part
+                columns_work = build_columns_work(*zip(*column_seqs), columns_part, columns_route)
         if tile_prefill:
             for b in range(B):
                 n, c = int(qlens[b]), int(ctx[b])
@@ -542,6 +572,9 @@ def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, bl
         prefill_max_tiles=prefill_tiles_max,
         columns_work_np=columns_work,
         num_columns_work=0 if columns_work is None else int(columns_work.shape[0]),
+        columns_route=None if columns_work is None else columns_route,
+        columns_seqs=column_seqs or None,
+        columns_partition=columns_part,
         superseded=bool(np.any((slots < 0) & (row_ctx_by_row > 0))),
     )
 

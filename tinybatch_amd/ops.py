@@ -595,10 +595,11 @@ def paged_attention(q: torch.Tensor, pool: torch.Tensor, meta: StepMetadata, *, 
             raise ValueError("noalloc takes no workspace")
         if workspace is None and not noalloc:
             workspace = workspace_for(meta, num_heads, d, q.device)
+        columns, num_columns = meta.columns_for(num_heads, hkv, q.device)
         last = not meta.num_work_items and not meta.num_prefill_tiles
         _lib.check(_lib.lib().tb_paged_prefill_columns(
             q.data_ptr(), qs, pool.data_ptr(), nb, out.data_ptr(), os_, meta.block_tables.data_ptr(),
-            meta.max_blocks_per_seq, meta.columns_work.data_ptr(), meta.num_columns_work, meta.row_part_off.data_ptr(), T,
+            meta.max_blocks_per_seq, columns.data_ptr(), num_columns, meta.row_part_off.data_ptr(), T,
             meta.split_rows.data_ptr(), meta.num_split_rows if last else 0, meta.max_parts_per_row,
             meta.total_partitions, num_heads, hkv, d, bs, float(scale), _lib.DTYPE_CODE[q.dtype],
             None if workspace is None else workspace.data_ptr(),
