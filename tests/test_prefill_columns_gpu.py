@@ -138,3 +138,15 @@ def test_metadata_of_other_heads(Hq, Hkv, monkeypatch):
         got = ops.paged_attention(q, pool, meta, num_heads=Hq, out=out).cpu()
         torch.testing.assert_close(got.float(), want.float(), **TOL)
     assert len(meta.columns_other) == 1
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,dtype", [(14, 2, 64, torch.bfloat16), (32, 8, 128, torch.float16),
+                                            (14, 2, 64, torch.float32), (32, 8, 128, torch.float32)])
+@pytest.mark.parametrize("sign", [-1, 0])
+def test_negative_and_zero_scale(Hq, Hkv, D, dtype, sign):
+    """The scores of -q at the scale's size, or uniform weights: masked positions stay masked."""
+    c = case(11, Hq, Hkv, D, 16, dtype, [70, 20], [200, 0])
+    want = ref.attention(sign * c["q"], c["pool"], c["slices"], c["tables"], c["ctx"], Hq, Hkv)
+    got = ops.paged_attention(c["q"].to(DEV), c["pool"].to(DEV), metadata(c), num_heads=Hq, scale=sign * D ** -0.5)
+    torch.testing.assert_close(got.cpu().float(), want.float(),
+                               **(dict(atol=1e-5, rtol=0) if dtype == torch.float32 else TOL))

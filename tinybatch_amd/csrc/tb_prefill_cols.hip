@@ -37,6 +37,7 @@
 // chunk's loads spread between its products (the same); row sums on the matrix unit (5%
 // slower at head dim 64).
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "tb_stream.h"
@@ -88,7 +89,8 @@ struct cols_args {
   float* ws_ml;                // [parts][Hq][2]
   int32_t num_heads, num_kv_heads, rep;
   int32_t log2_bs;             // block size: a power of two >= 16
-  float scale_log2e;
+  float scale_log2e;           // > 0: the scale's size times log2(e), or 1 for a scale of 0
+  float q_sign;                // 1, -1 or 0 (NaN: a NaN scale): multiplies q, so that masked scores stay -inf
   rope_tables rope;
 };
 
@@ -206,6 +208,15 @@ __global__ __launch_bounds__(64 * cshape<D>::NW * SP, 2) void paged_prefill_colu
 #pragma unroll
     for (int s = 0; s < KS / 2; ++s)            // slices s and s + KS/2 pair (dims i and i + D/2)
       rope_pair<scalar_t>(qv[s], qv[s + KS / 2], a.rope.cos + r + 16 * s, a.rope.sin + r + 16 * s);
+  }
+  if (a.q_sign != 1.f) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      typename M::vec8_t x = __builtin_bit_cast(typename M::vec8_t, qv[s]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = (scalar_t)((float)x[e] * a.q_sign);
+      qv[s] = __builtin_bit_cast(vec16, x);
+    }
   }
   su32x4_t q[KS];
 #pragma unroll
@@ -506,6 +517,12 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void paged_prefill_columns_f3
 #pragma unroll
     for (int c = 0; c < KC / 2; ++c)
       rope_pair<float>(q[c], q[c + KC / 2], a.rope.cos + r + 8 * c, a.rope.sin + r + 8 * c);
+  }
+  if (a.q_sign != 1.f) {
+#pragma unroll
+    for (int c = 0; c < KC; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) q[c].w[i] = __float_as_uint(bits_to_f32(q[c].w[i]) * a.q_sign);
   }
 #pragma unroll
   for (int c = 0; c < KC; ++c)
@@ -843,7 +860,8 @@ extern "C" int32_t tb_paged_prefill_columns(const void* q, int64_t q_row_stride,
   a.num_kv_heads = num_kv_heads;
   a.rep = num_heads / num_kv_heads;
   while ((1 << a.log2_bs) < block_size) ++a.log2_bs;
-  a.scale_log2e = scale * 1.4426950408889634f;
+  a.scale_log2e = scale > 0.f || scale < 0.f ? fabsf(scale) * 1.4426950408889634f : 1.f;
+  a.q_sign = scale > 0.f ? 1.f : scale < 0.f ? -1.f : scale * 0.f;
   a.rope = rope_tables{rope_cos, rope_sin, rope_max_position};
   const bool d64 = head_dim == 64;
   if (dtype == TB_DTYPE_F32) {
