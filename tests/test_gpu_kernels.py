@@ -449,3 +449,14 @@ def test_mixed_step_one_launch_tiles_and_decode_items(BS, dtype):
     wave-uniform tiles); tolerance 2e-2 against the oracle."""
     c = _mixed_case(41 + BS, 14, 2, 64, BS, dtype, qlens=[40, 1, 1, 100, 33, 1], cached=[0, 300, 2000, 200, 700, 17])
     _attention_vs_oracle(c, 14, 2, dtype)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,rows", [(14, 2, 64, 3), (14, 2, 64, 130), (32, 8, 128, 3), (64, 8, 128, 40)])
+def test_fp32_scores_of_minus_infinity(Hq, Hkv, D, rows):
+    """16 positions whose scores are all -inf weigh nothing (a wave's whole share of a step)."""
+    c = _mixed_case(12, Hq, Hkv, D, 16, torch.float32, qlens=[1] * rows, cached=[70 + r % 5 for r in range(rows)])
+    c["q"][:, :, 0] = 1.0
+    for t in c["tables"]:
+        c["pool"][t[0], 0, :, :, 0] = float("-inf")
+        c["pool"][t[2], 0, :, :, 0] = float("-inf")
+    _attention_vs_oracle(c, Hq, Hkv, torch.float32)

@@ -233,15 +233,15 @@ __global__ __launch_bounds__(64 * NW_) void paged_attn_f32_kernel(const attn_arg
 #pragma unroll
     for (int j = 0; j < 4; ++j) s[j] = vpos + j < p1 ? s[j] * a.scale_log2e : -INFINITY;
     const float cm = max_xor32(max_xor16(max_f32(max_f32(s[0], s[1]), max_f32(s[2], s[3]))));
-    const float m_new = max_f32(m, cm);    // finite: the tile's first position is visible
-    const float alpha = fast_exp2(m - m_new);
+    const float m_new = max_f32(m, cm), m_safe = m_new == -INFINITY ? 0.f : m_new;   // every score so far -inf
+    const float alpha = fast_exp2(m - m_safe);         // 0 while m = -inf
     m = m_new;
     l *= alpha;
 #pragma unroll
     for (int e = 0; e < 4 * VC; ++e) acc[e] *= alpha;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float p = fast_exp2(s[j] - m);
+      const float p = fast_exp2(s[j] - m_safe);
       l += p;
       const bool seen = vpos + j < p1;     // what stands in for a row past the context counts as zeros
 #pragma unroll
