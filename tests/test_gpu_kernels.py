@@ -460,3 +460,20 @@ def test_fp32_scores_of_minus_infinity(Hq, Hkv, D, rows):
         c["pool"][t[0], 0, :, :, 0] = float("-inf")
         c["pool"][t[2], 0, :, :, 0] = float("-inf")
     _attention_vs_oracle(c, Hq, Hkv, torch.float32)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(64, 8, 128), (15, 1, 128), (14, 1, 64), (16, 1, 128), (16, 1, 64)])
+@pytest.mark.parametrize("rows", [2, 70])
+def test_fp32_heads_of_a_workgroup(Hq, Hkv, D, rows):
+    """8, 15 and 14 heads on one workgroup (the widest merges in LDS), 16 on two of 8, of
+    which one stores the appended row; few work items (8 or 16 waves each) and many (4)."""
+    c = _mixed_case(13, Hq, Hkv, D, 16, torch.float32, qlens=[1] * rows, cached=[250 + 9 * (r % 40) for r in range(rows)])
+    g = torch.Generator().manual_seed(rows)
+    k, v = (torch.randn(rows, Hkv, D, generator=g) for _ in range(2))
+    pool = c["pool"].clone()
+    want = ref.decode_step(pool, c["q"], k, v, [n - 1 for n in c["ctx"]], c["tables"], Hq, Hkv, 16)
+    got_pool = c["pool"].to(DEV)
+    meta = _meta(c["pos"], c["slices"], c["tables"], c["ctx"], 16, c["NB"])
+    out = ops.paged_attention(c["q"].to(DEV), got_pool, meta, num_heads=Hq, k_new=k.to(DEV), v_new=v.to(DEV))
+    torch.testing.assert_close(out.cpu(), want, **TOL[torch.float32])
+    assert torch.equal(got_pool.cpu(), pool)

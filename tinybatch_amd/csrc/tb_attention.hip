@@ -125,6 +125,8 @@ struct f32_shape {
   static constexpr int NW = NW_;           // waves per workgroup
   static constexpr int SPAN = 16 * NW;     // positions in flight
   static constexpr int PITCH = D + 4;      // floats per (wave, head) row of the merge
+  // heads whose merge fits 64 KiB beside the waves' (max, sum) pairs: 14 or 15
+  static constexpr int max_heads = (65536 / (NW * (int)sizeof(float)) - 32) / PITCH;
 };
 
 template <int D, int NW_>
@@ -1290,7 +1292,9 @@ static int32_t paged_attention_impl(const void* q, int64_t q_row_stride, void* p
 
   const int rep = num_heads / num_kv_heads;
   // heads per workgroup: the MFMA operand holds 16; the fp32 kernel's merge keeps to 64 KiB of LDS
-  const int group = largest_divisor_upto(rep, eb == 2 ? 16 : head_dim == 64 ? 14 : 7);
+  // (16 waves at head dim 64, 8 at 128: f32_shape::max_heads)
+  const int group = largest_divisor_upto(rep, eb == 2 ? 16 : head_dim == 64 ? f32_shape<64, 16>::max_heads
+                                                                            : f32_shape<128, 8>::max_heads);
   const bool merged = slot_map != nullptr;
   if (merged) {   // split rows merged inside the launch of the 16-bit work-item kernel
     if (eb != 2 || num_prefill_tiles > 0 || group != rep || device_counts) return TB_ERR_UNSUPPORTED;

@@ -124,7 +124,9 @@ def kv_gather(pool: torch.Tensor, table: torch.Tensor, context_len: int) -> tupl
 
 
 def heads_per_group(dtype: torch.dtype, num_heads: int, num_kv_heads: int) -> int:
-    """Query heads one work item serves (the C dispatch uses the same rule)."""
+    """Query heads one 16-bit work item serves (the C dispatch uses the same rule). fp32
+    items serve one row whatever the number of heads; the C dispatch puts up to 14 (head
+    dim 64) or 15 (128) heads of it on a workgroup."""
     rep = num_heads // num_kv_heads
     cap = 16 if dtype in (torch.float16, torch.bfloat16) else 8
     return max(t for t in range(1, cap + 1) if rep % t == 0)
