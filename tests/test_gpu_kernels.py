@@ -10,9 +10,10 @@ import pytest
 import torch
 
 from oracle import reference_path as ref
-from tinybatch_amd import ops
+from tinybatch_amd import layer_ops, ops
 from tinybatch_amd.kv_cache import PagedKVCache
 from tinybatch_amd.metadata import build_step_metadata
+from tinybatch_amd.model import rope_tables
 from tinybatch_amd.workloads import make_decode_workload
 
 pytestmark = pytest.mark.gpu
@@ -475,5 +476,35 @@ def test_fp32_heads_of_a_workgroup(Hq, Hkv, D, rows):
     got_pool = c["pool"].to(DEV)
     meta = _meta(c["pos"], c["slices"], c["tables"], c["ctx"], 16, c["NB"])
     out = ops.paged_attention(c["q"].to(DEV), got_pool, meta, num_heads=Hq, k_new=k.to(DEV), v_new=v.to(DEV))
+    torch.testing.assert_close(out.cpu(), want, **TOL[torch.float32])
+    assert torch.equal(got_pool.cpu(), pool)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(8, 8, 64), (8, 4, 128), (12, 4, 64), (16, 4, 128), (20, 4, 64), (32, 8, 64),
+                                      (28, 4, 128), (64, 8, 64)])
+@pytest.mark.parametrize("per_head", [318, 322, 126, 130])
+def test_fp32_many_items_of_few_heads(Hq, Hkv, D, per_head):
+    """1 to 8 heads on a workgroup, either side of 320 workgroups a head (128 where no table
+    holds more than 64 positions), with the fused append and RoPE, split rows, contexts
+    around the chunks of both kernels."""
+    rep, line = Hq // Hkv, 320 if per_head > 200 else 128
+    items = per_head * rep // Hkv if per_head < line else -(-per_head * rep // Hkv)
+    longer = [300, 511, 256] if line == 320 else []                # 2 partitions each
+    cached = [[3, 15, 16, 31, 32, 60][r % 6] for r in range(items - 2 * len(longer))] + longer
+    rows = len(cached)
+    c = _mixed_case(14, Hq, Hkv, D, 16, torch.float32, qlens=[1] * rows, cached=cached)
+    meta = _meta(c["pos"], c["slices"], c["tables"], c["ctx"], 16, c["NB"])
+    assert (meta.num_work_items * Hkv >= line * rep) == (per_head > line)
+    g = torch.Generator().manual_seed(rows)
+    k, v = (torch.randn(rows, Hkv, D, generator=g) for _ in range(2))
+    cos, sin = rope_tables(D, 1e6, 1024, DEV)
+    pos = torch.tensor(c["pos"], device=DEV)
+    qkv = torch.cat([c["q"].to(DEV), k.to(DEV), v.to(DEV)], 1).reshape(rows, -1)
+    rq, rk = layer_ops.rope_qk(qkv, pos, cos, sin, Hq, Hkv, D)
+    pool = c["pool"].clone()
+    want = ref.decode_step(pool, rq.cpu(), rk.cpu(), v, [n - 1 for n in c["ctx"]], c["tables"], Hq, Hkv, 16)
+    got_pool = c["pool"].to(DEV)
+    out = ops.paged_attention(c["q"].to(DEV), got_pool, meta, num_heads=Hq, k_new=k.to(DEV), v_new=v.to(DEV),
+                              rope=ops.Rope(cos, sin))
     torch.testing.assert_close(out.cpu(), want, **TOL[torch.float32])
     assert torch.equal(got_pool.cpu(), pool)

@@ -29,7 +29,8 @@
 // workgroup per (64 query rows of one sequence, query head) that walks the
 // causal range in 64-position chunks staged in LDS (see the kernel).
 // fp32: paged_attn_f32_kernel, the fp32 MFMA (fp32 products and sums), same
-// decomposition with one query row per item.
+// decomposition with one query row per item; paged_attn_valu_kernel (fp32 FMAs) for
+// many items of few heads.
 // Positions >= the row's context are never loaded from the pool (stale slots
 // may hold any bits, NaN included): their scores are -inf, so p = 0, and what
 // stands in for their V rows is finite.
@@ -300,6 +301,216 @@ __global__ __launch_bounds__(64 * NW_) void paged_attn_f32_kernel(const attn_arg
       if (d4 == 0) *reinterpret_cast<float2*>(a.ws_ml + pidx * 2) = make_float2(M, L);
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// fp32 path, many items of few heads (launch_f32): a wave per work item walks its partition 32
+// (head dim 64) or 16 positions at a time, fp32 FMAs on the VALU reduced across lanes, online
+// softmax per chunk. No matrix columns are spent on heads that are not there, and one wave an
+// item leaves room for many items on a CU: us per layer against the kernel above, 200 rows of
+// up to 40 positions at 8 / 8 heads of 64: 10.4 (16.1); of up to 2500: 309 (346); at 32 / 8
+// heads of 128: 18.8 (28.2) and 645 (694).
+template <typename Tag, int D>
+struct valu_shape {
+  static constexpr int EB = elem<Tag>::bytes;
+  static constexpr int EPL = 16 / EB;     // elements per lane per load
+  static constexpr int LPT = D / EPL;     // lanes per token row
+  static constexpr int TPL = 64 / LPT;    // tokens per wave load
+  static constexpr int CH_LOADS = 8;      // wave loads of K (and of V) per chunk
+  static constexpr int CH = CH_LOADS * TPL;  // tokens per chunk
+  static_assert(LPT >= 1 && LPT <= 64 && (64 % LPT) == 0, "lane split");
+};
+
+// End of a VALU work item. acc[h][e] holds, in lanes 0..LPT-1 (column j = lane),
+// the unnormalised output of head h over the partition for dims j*EPL..;
+// m[h] / l[h] (wave-uniform) are its max (base-2 domain) and sum. One
+// partition: write the output. Several: write the partial for the combine.
+template <typename Tag, int D, int REP, int EPL, int LPT>
+__device__ __forceinline__ void finish_valu(const attn_args& a, int row, int part, int head0, int lane,
+                                            float (&acc)[REP][EPL], const float (&m)[REP],
+                                            const float (&l)[REP]) {
+  const int j = lane % LPT;
+  if (lane >= LPT) return;
+  const int pbeg = a.row_part_off[row];
+  const int nparts = a.row_part_off[row + 1] - pbeg;
+  if (nparts == 1) {
+    char* orow = a.out + row * a.out_row_bytes + j * 16;
+#pragma unroll
+    for (int h = 0; h < REP; ++h) {
+      const float inv = 1.f / l[h];
+      vec16 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o.w[e] = __float_as_uint(acc[h][e] * inv);
+      st16_through(orow + (int64_t)(head0 + h) * D * 4, o);
+    }
+    return;
+  }
+  const int64_t pidx = pbeg + part;
+#pragma unroll
+  for (int h = 0; h < REP; ++h) {
+    float* dst = a.ws_acc + (pidx * a.num_heads + head0 + h) * D + j * EPL;
+#pragma unroll
+    for (int e = 0; e < EPL; e += 4)
+      *reinterpret_cast<float4*>(dst + e) = make_float4(acc[h][e], acc[h][e + 1], acc[h][e + 2], acc[h][e + 3]);
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int h = 0; h < REP; ++h)
+      *reinterpret_cast<float2*>(a.ws_ml + (pidx * a.num_heads + head0 + h) * 2) = make_float2(m[h], l[h]);
+  }
+}
+
+template <typename Tag, int D, int REP>
+__global__ __launch_bounds__(64) void paged_attn_valu_kernel(const attn_args a) {
+  using S = valu_shape<Tag, D>;
+  constexpr int EB = S::EB, EPL = S::EPL, LPT = S::LPT, TPL = S::TPL;
+  constexpr int CH_LOADS = S::CH_LOADS, CH = S::CH;
+  static_assert(EB == 4, "the 16-bit types use paged_attn_mfma_kernel");
+
+  const int lane = threadIdx.x;
+  const int j = lane % LPT;  // 16-byte column of the token row
+  const int g = lane / LPT;  // token slot inside one wave load
+
+  const int4 wi = a.work[blockIdx.x];   // one row per item on this path; the array holds the grid's capacity
+  if (a.counts && (int)blockIdx.x >= a.counts[0]) return;   // beyond this step's work items
+  const int row = wi.x, seq = wi.y, part = wi.z & 0xFFFFFF, ctx = wi.w;
+  const int kvh = blockIdx.y;
+  const int head0 = kvh * a.rep + blockIdx.z * REP;
+
+  const int p0 = part * a.part_tokens;
+  const int p1 = min(p0 + a.part_tokens, ctx);
+  const int bs = 1 << a.log2_bs;
+
+  // Block-table entries of this partition: lane l holds entry p0/BS + l.
+  const int blk_first = p0 >> a.log2_bs;
+  const int blk_count = ((p1 - 1) >> a.log2_bs) - blk_first + 1;  // <= 64 (host-checked)
+  int my_blk = 0;
+  if (lane < blk_count) {
+    my_blk = a.block_tables[(int64_t)seq * a.max_nb + blk_first + lane];
+    if (my_blk < 0 || my_blk >= a.num_blocks) my_blk = 0;  // host validates; stay inside the pool
+  }
+
+  const int64_t tile_bytes = (int64_t)bs * D * EB;
+  const int64_t blk_bytes = 2 * (int64_t)a.num_kv_heads * tile_bytes;
+  const int64_t v_off = (int64_t)a.num_kv_heads * tile_bytes;
+  const char* pool_kvh = a.pool + kvh * tile_bytes + j * 16;
+  const int new_pos = ctx - 1;
+  const bool fused = (a.k_new != nullptr);
+  const char* k_new_row = fused ? a.k_new + row * a.k_new_row_bytes + (int64_t)kvh * D * EB + j * 16 : nullptr;
+  const char* v_new_row = fused ? a.v_new + row * a.v_new_row_bytes + (int64_t)kvh * D * EB + j * 16 : nullptr;
+
+  vec16 qv[REP];
+  {
+    const char* qrow = a.q + row * a.q_row_bytes + j * 16;
+#pragma unroll
+    for (int h = 0; h < REP; ++h) qv[h] = ld16(qrow + (int64_t)(head0 + h) * D * EB);
+  }
+  // RoPE: chunk j of the first half pairs with chunk j + LPT/2 of the second,
+  // held by lane ^ LPT/2 of the same token slot (every lane holds its chunk)
+  vec16 k_new_rot = zero16();
+  if (a.rope.cos) {
+    const bool first = j < LPT / 2;
+    const int64_t r = a.rope.row(ctx - 1, D / 2) + (first ? j : j - LPT / 2) * 4;
+    auto rotate = [&](vec16& x) {
+      vec16 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y.w[e] = (uint32_t)__shfl_xor((int)x.w[e], LPT / 2);
+      if (first) rope_pair<float>(x, y, a.rope.cos + r, a.rope.sin + r);
+      else rope_pair<float>(y, x, a.rope.cos + r, a.rope.sin + r);
+    };
+#pragma unroll
+    for (int h = 0; h < REP; ++h) rotate(qv[h]);
+    if (fused) {
+      k_new_rot = ld16(k_new_row);
+      rotate(k_new_rot);
+    }
+  }
+
+  float m_run[REP], l_run[REP], acc[REP][EPL];
+#pragma unroll
+  for (int h = 0; h < REP; ++h) {
+    m_run[h] = -INFINITY;
+    l_run[h] = 0.f;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) acc[h][e] = 0.f;
+  }
+
+  int64_t new_off = 0;
+  if (fused) {
+    const int nb = __shfl(my_blk, ((new_pos - p0) >> a.log2_bs) & 63);
+    new_off = (int64_t)nb * blk_bytes + (int64_t)(new_pos & (bs - 1)) * (D * EB);
+  }
+
+  for (int c0 = p0; c0 < p1; c0 += CH) {
+    vec16 kbuf[CH_LOADS], vbuf[CH_LOADS];
+#pragma unroll
+    for (int i = 0; i < CH_LOADS; ++i) {
+      const int tau = c0 + i * TPL + g;
+      const int blk = __shfl(my_blk, ((tau - p0) >> a.log2_bs) & 63);
+      const int64_t off = (int64_t)blk * blk_bytes + (int64_t)(tau & (bs - 1)) * (D * EB);
+      const char* kp = pool_kvh + off;
+      const char* vp = kp + v_off;
+      if (fused && tau == new_pos) { kp = k_new_row; vp = v_new_row; }
+      if (tau < p1) { kbuf[i] = ld16(kp); vbuf[i] = ld16(vp); }
+      else { kbuf[i] = zero16(); vbuf[i] = zero16(); }
+      if (fused && a.rope.cos && tau == new_pos) kbuf[i] = k_new_rot;
+    }
+    if (fused) {
+#pragma unroll
+      for (int i = 0; i < CH_LOADS; ++i) {
+        if (c0 + i * TPL + g == new_pos) {
+          char* kp = const_cast<char*>(pool_kvh) + new_off;
+          st16_through(kp, kbuf[i]);
+          st16_through(kp + v_off, vbuf[i]);
+        }
+      }
+    }
+    float s[CH_LOADS][REP];
+#pragma unroll
+    for (int i = 0; i < CH_LOADS; ++i) {
+      const bool valid = (c0 + i * TPL + g) < p1;
+#pragma unroll
+      for (int h = 0; h < REP; ++h) {
+        float d = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d = fmaf(bits_to_f32(qv[h].w[e]), bits_to_f32(kbuf[i].w[e]), d);
+        d = group_sum<LPT>(d);
+        s[i][h] = valid ? d * a.scale_log2e : -INFINITY;
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < REP; ++h) {
+      float cm = s[0][h];
+#pragma unroll
+      for (int i = 1; i < CH_LOADS; ++i) cm = fmaxf(cm, s[i][h]);
+      cm = cross_group_max<LPT>(cm);
+      const float m_new = fmaxf(m_run[h], cm);
+      const float alpha = fast_exp2(m_run[h] - m_new);
+      m_run[h] = m_new;
+      l_run[h] *= alpha;
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) acc[h][e] *= alpha;
+    }
+#pragma unroll
+    for (int i = 0; i < CH_LOADS; ++i) {
+#pragma unroll
+      for (int h = 0; h < REP; ++h) {
+        const float p = fast_exp2(s[i][h] - m_run[h]);
+        l_run[h] += p;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[h][e] = fmaf(p, bits_to_f32(vbuf[i].w[e]), acc[h][e]);
+      }
+    }
+  }
+
+  // l was accumulated per token slot; sum over the slots like acc
+#pragma unroll
+  for (int h = 0; h < REP; ++h) {
+    l_run[h] = cross_group_sum<LPT>(l_run[h]);
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) acc[h][e] = cross_group_sum<LPT>(acc[h][e]);
+  }
+  finish_valu<Tag, D, REP, EPL, LPT>(a, row, part, head0, lane, acc, m_run, l_run);
 }
 
 // ---------------------------------------------------------------------------
@@ -1102,6 +1313,12 @@ __global__ __launch_bounds__(COMBINE_THREADS) void combine_partials_kernel(const
 }
 
 // ---- dispatch ---------------------------------------------------------------
+template <typename Tag, int D, int REP>
+static void launch_valu(const attn_args& a, int num_work, hipStream_t stream) {
+  hipLaunchKernelGGL((paged_attn_valu_kernel<Tag, D, REP>), dim3(num_work, a.num_kv_heads, a.rep / a.group),
+                     dim3(64), 0, stream, a);
+}
+
 template <int D, int NW>
 static void launch_f32_nw(const attn_args& a, int num_work, hipStream_t stream) {
   using S = f32_shape<D, NW>;
@@ -1111,15 +1328,38 @@ static void launch_f32_nw(const attn_args& a, int num_work, hipStream_t stream) 
 }
 
 // A step of few work items is a chain of latencies: a whole partition in flight (16 waves; 8
-// at head dim 128, whose registers do not fit 16). From 256 workgroups on (one per CU)
-// four waves: more workgroups on a CU hide the chain better than more waves on an item.
+// at head dim 128, whose registers do not fit 16). From 256 workgroups on (one per CU), and
+// where the tables hold 64 positions at most, four waves: more workgroups on a CU hide the
+// chain better than more waves on an item.
+// From 320 workgroups per head on, up to five heads: the VALU kernel, whose work grows with
+// the heads while the matrix unit does 16 whatever there are. us per layer, VALU against
+// matrix unit, head dim 64 unless said: 1 head, 288 workgroups 18.3 / 18.5, 576: 19.5 / 22.5;
+// 2 heads, 576: 21.9 / 20.8, 1200: 33.0 / 39.2; 4 heads, 868: 36.8 / 34.3, 1740: 50.1 / 54.9 (128:
+// 1152: 70.1 / 64.6, 1736: 85.0 / 98.8); 5 heads, 1200: 44.8 / 39.9, 1740: 52.5 / 55.7; 6 heads,
+// 1740 at 128: 103 / 100; 7 heads, 1830: 61.8 / 57.8. With 64 positions at most, where most of a
+// matrix wave's positions are not there, from 128 per head on, up to eight heads (128, up to
+// 40 positions: 4 heads, 384: 12.8 / 10.8, 800: 14.9 / 18.2; 8 heads, 800: 20.8 / 18.9, 1600: 26.8 / 30.0).
 template <int D>
 static void launch_f32(const attn_args& a, int num_work, hipStream_t stream) {
   if (num_work <= 0) return;
-  if ((int64_t)num_work * a.num_kv_heads * (a.rep / a.group) < 256)
+  const int64_t wgs = (int64_t)num_work * a.num_kv_heads * (a.rep / a.group);
+  const bool brief = ((int64_t)a.max_nb << a.log2_bs) <= 64;
+  if (a.group <= (brief ? 8 : 5) && wgs >= (brief ? 128 : 320) * a.group) {
+    switch (a.group) {
+      case 1: launch_valu<f32_t, D, 1>(a, num_work, stream); break;
+      case 2: launch_valu<f32_t, D, 2>(a, num_work, stream); break;
+      case 3: launch_valu<f32_t, D, 3>(a, num_work, stream); break;
+      case 4: launch_valu<f32_t, D, 4>(a, num_work, stream); break;
+      case 5: launch_valu<f32_t, D, 5>(a, num_work, stream); break;
+      case 6: launch_valu<f32_t, D, 6>(a, num_work, stream); break;
+      case 7: launch_valu<f32_t, D, 7>(a, num_work, stream); break;
+      default: launch_valu<f32_t, D, 8>(a, num_work, stream); break;
+    }
+  } else if (wgs < 256 && !brief) {
     launch_f32_nw<D, D == 64 ? 16 : 8>(a, num_work, stream);
-  else
+  } else {
     launch_f32_nw<D, 4>(a, num_work, stream);
+  }
 }
 
 template <typename Tag, int D>

@@ -114,6 +114,65 @@ template <> struct elem<bf16_t> {
 __device__ __forceinline__ float bits_to_f32(uint32_t u) { return __uint_as_float(u); }
 
 // ---- cross-lane helpers ---------------------------------------------------
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false));
+}
+
+// DPP control words (GCN/CDNA encoding).
+constexpr int DPP_QUAD_XOR1 = 0xB1;        // quad_perm [1,0,3,2]
+constexpr int DPP_QUAD_XOR2 = 0x4E;        // quad_perm [2,3,0,1]
+constexpr int DPP_ROW_HALF_MIRROR = 0x141; // lane i <- lane 7-i inside each 8-lane half row
+constexpr int DPP_ROW_MIRROR = 0x140;      // lane i <- lane 15-i inside each 16-lane row
+constexpr int DPP_ROW_ROR8 = 0x128;        // lane i <- lane (i+8)%16 inside a row, i.e. xor 8
+
+// Sum over aligned groups of N consecutive lanes; every lane of a group ends
+// with the group total. Pairings: xor1, xor2, then mirrors, which pair each
+// lane with a lane of the other half once the halves are already reduced.
+template <int N>
+__device__ __forceinline__ float group_sum(float x) {
+  static_assert(N == 1 || N == 2 || N == 4 || N == 8 || N == 16 || N == 32 || N == 64, "group");
+  if constexpr (N >= 2) x += dpp<DPP_QUAD_XOR1>(x);
+  if constexpr (N >= 4) x += dpp<DPP_QUAD_XOR2>(x);
+  if constexpr (N >= 8) x += dpp<DPP_ROW_HALF_MIRROR>(x);
+  if constexpr (N >= 16) x += dpp<DPP_ROW_MIRROR>(x);
+  if constexpr (N >= 32) x += __shfl_xor(x, 16);
+  if constexpr (N >= 64) x += __shfl_xor(x, 32);
+  return x;
+}
+
+template <int MASK>
+__device__ __forceinline__ float lane_xor(float x) {
+  if constexpr (MASK == 1) return dpp<DPP_QUAD_XOR1>(x);
+  else if constexpr (MASK == 2) return dpp<DPP_QUAD_XOR2>(x);
+  else if constexpr (MASK == 8) return dpp<DPP_ROW_ROR8>(x);
+  else return __shfl_xor(x, MASK);
+}
+
+// Reduce across lanes that differ only in the bits >= FIRST (lane groups of
+// FIRST consecutive lanes hold the same "column"): max and sum variants.
+template <int FIRST>
+__device__ __forceinline__ float cross_group_max(float x) {
+  if constexpr (FIRST <= 1) x = fmaxf(x, lane_xor<1>(x));
+  if constexpr (FIRST <= 2) x = fmaxf(x, lane_xor<2>(x));
+  if constexpr (FIRST <= 4) x = fmaxf(x, lane_xor<4>(x));
+  if constexpr (FIRST <= 8) x = fmaxf(x, lane_xor<8>(x));
+  if constexpr (FIRST <= 16) x = fmaxf(x, lane_xor<16>(x));
+  if constexpr (FIRST <= 32) x = fmaxf(x, lane_xor<32>(x));
+  return x;
+}
+
+template <int FIRST>
+__device__ __forceinline__ float cross_group_sum(float x) {
+  if constexpr (FIRST <= 1) x += lane_xor<1>(x);
+  if constexpr (FIRST <= 2) x += lane_xor<2>(x);
+  if constexpr (FIRST <= 4) x += lane_xor<4>(x);
+  if constexpr (FIRST <= 8) x += lane_xor<8>(x);
+  if constexpr (FIRST <= 16) x += lane_xor<16>(x);
+  if constexpr (FIRST <= 32) x += lane_xor<32>(x);
+  return x;
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // gfx950 LDS transpose read (ds_read_b64_tr_b16). Within each group of 16
