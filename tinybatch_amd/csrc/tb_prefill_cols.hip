@@ -646,7 +646,7 @@ bool columns_args_ok(const int32_t* pos0, const int32_t* new_rows, int32_t num_s
   if (num_seqs < 0 || num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads) return false;
   if (num_seqs > 0 && (!pos0 || !new_rows)) return false;
   for (int i = 0; i < num_seqs; ++i)
-    if (pos0[i] < 0 || new_rows[i] <= 0 || (int64_t)pos0[i] + new_rows[i] > (1 << 24) ||
+    if (pos0[i] < 0 || new_rows[i] <= 0 || (int64_t)pos0[i] + new_rows[i] > (1 << 30) ||
         (int64_t)new_rows[i] * (num_heads / num_kv_heads) > (1 << 28))
       return false;
   return true;
@@ -656,6 +656,31 @@ bool columns_args_ok(const int32_t* pos0, const int32_t* new_rows, int32_t num_s
 int columns_limit(int pos0, int new_rows, int rep, int col0) {
   return pos0 + std::min(col0 + COLS - 1, new_rows * rep - 1) / rep + 1;
 }
+
+// The column tiles of a step by their chunks: reach[n - 1] tiles (of one kv head) have n or
+// more, so that a partition length is priced in longest / length steps.
+struct column_tiles {
+  std::vector<int32_t> reach;
+  int64_t chunks = 0;
+  int longest = 0;
+
+  column_tiles(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs, int rep) {
+    auto each = [&](auto&& f) {
+      for (int i = 0; i < num_seqs; ++i)
+        for (int c = 0; c < new_rows[i] * rep; c += COLS)
+          f((columns_limit(pos0[i], new_rows[i], rep, c) + CHUNK - 1) / CHUNK);
+    };
+    each([&](int n) { longest = std::max(longest, n); });
+    reach.assign(longest + 1, 0);
+    each([&](int n) { ++reach[n - 1], chunks += n; });
+    for (int n = longest - 1; n > 0; --n) reach[n - 1] += reach[n];
+  }
+  int64_t entries(int part) const {   // of `part` chunks or fewer
+    int64_t n = 0;
+    for (int64_t at = 0; at < longest; at += part) n += reach[at];
+    return n;
+  }
+};
 
 }  // namespace
 
@@ -667,14 +692,8 @@ extern "C" int32_t tb_prefill_columns_partition(const int32_t* pos0, const int32
   if ((head_dim != 64 && head_dim != 128) || (dtype != TB_DTYPE_F32 && dtype != TB_DTYPE_F16 && dtype != TB_DTYPE_BF16))
     return TB_ERR_INVALID_ARG;
   const int rep = num_heads / num_kv_heads;
-  int64_t total = 0;
-  int longest = 0;
-  for (int i = 0; i < num_seqs; ++i)
-    for (int c = 0; c < new_rows[i] * rep; c += COLS) {
-      const int n = (columns_limit(pos0[i], new_rows[i], rep, c) + CHUNK - 1) / CHUNK;
-      total += (int64_t)n * num_kv_heads;
-      longest = std::max(longest, n);
-    }
+  const column_tiles tiles(pos0, new_rows, num_seqs, rep);
+  const int longest = tiles.longest;
   // The partition with the least cost, in us: a workgroup alone on its CU takes 1.0 (head
   // dim 64) or 1.6 us a chunk, a full CU 0.65 or 1.05 us per chunk of its workgroups (fp32, at
   // the matrix rate either way: 4 or 8 and 3.6 or 7.2); a split
@@ -684,12 +703,9 @@ extern "C" int32_t tb_prefill_columns_partition(const int32_t* pos0, const int32
   // 704 14.2 (16.9), one fresh prompt of 600 unsplit 16.8 (17.7).
   const bool d64 = head_dim == 64, f32 = dtype == TB_DTYPE_F32;
   const double alone = f32 ? (d64 ? 4.0 : 8.0) : d64 ? 1.0 : 1.6, full = f32 ? (d64 ? 3.6 : 7.2) : d64 ? 0.65 : 1.05;
-  const double share = full * (double)total / num_cus;
+  const double share = full * (double)(tiles.chunks * num_kv_heads) / num_cus;
   auto span = [&](int chunks) {
-    int64_t wgs = 0;
-    for (int i = 0; i < num_seqs; ++i)
-      for (int c = 0; c < new_rows[i] * rep; c += COLS)
-        wgs += ((columns_limit(pos0[i], new_rows[i], rep, c) + CHUNK - 1) / CHUNK + chunks - 1) / chunks * num_kv_heads;
+    const int64_t wgs = tiles.entries(chunks) * num_kv_heads;
     const double one = !f32 && wgs <= COLS_SHARED ? 0.66 * alone : alone;   // two sets of waves on its chunks
     return std::max(one * chunks, share + 0.5 * full * chunks);
   };
