@@ -281,6 +281,14 @@ int32_t tb_paged_prefill_columns(const void* q, int64_t q_row_stride, const void
 int32_t tb_prefill_columns_partition(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs,
                                      int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t dtype,
                                      int32_t num_cus, int32_t other_partitions);
+/* 1 where the column tiles serve a step's sequences of new_rows new rows from position pos0
+ * faster than tb_paged_attention does, 0 where it is the faster one, negative: a status code.
+ * tiles_served: whether that call gets 16-bit prefills as tiles (tb_build_step_metadata's
+ * rule) and not as work items; beside_others: whether the step has other rows, which share
+ * its launch. Host code, no device call. */
+int32_t tb_prefill_columns_pay(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs, int32_t num_heads,
+                               int32_t num_kv_heads, int32_t head_dim, int32_t dtype, int32_t num_cus,
+                               int32_t tiles_served, int32_t beside_others);
 /* The work list (host, no device call): *count entries of 8 int32 into work (work NULL: the
  * count alone). Entry g is meant for XCD g % num_xcds (1: placement unknown). */
 int32_t tb_build_prefill_columns_work(const int32_t* first_row, const int32_t* seq_index, const int32_t* pos0,

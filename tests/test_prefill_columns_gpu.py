@@ -14,6 +14,7 @@ from oracle import reference_path as ref
 from test_prefill_columns_work import both_routes
 from test_prefill_stream_gpu import DEV, TOL, case
 from tinybatch_amd import layer_ops, ops
+from tinybatch_amd.kv_cache import PagedKVCache
 from tinybatch_amd.metadata import TILE_PARTITION, build_step_metadata
 from tinybatch_amd.model import rope_tables
 
@@ -148,5 +149,24 @@ def test_negative_and_zero_scale(Hq, Hkv, D, dtype, sign):
     c = case(11, Hq, Hkv, D, 16, dtype, [70, 20], [200, 0])
     want = ref.attention(sign * c["q"], c["pool"], c["slices"], c["tables"], c["ctx"], Hq, Hkv)
     got = ops.paged_attention(c["q"].to(DEV), c["pool"].to(DEV), metadata(c), num_heads=Hq, scale=sign * D ** -0.5)
+    torch.testing.assert_close(got.cpu().float(), want.float(),
+                               **(dict(atol=1e-5, rtol=0) if dtype == torch.float32 else TOL))
+
+
+@pytest.mark.parametrize("dtype,qlens,cached,columns", [(torch.bfloat16, [40, 1, 1], [0, 300, 700], False),
+                                                        (torch.bfloat16, [700, 3], [0, 50], False),
+                                                        (torch.bfloat16, [1500] * 4 + [1], [0] * 4 + [200], True),
+                                                        (torch.float32, [20, 1], [100, 300], False),
+                                                        (torch.float32, [300] * 6, [0] * 6, True)])
+def test_cache_takes_the_faster_route(dtype, qlens, cached, columns):
+    """PagedKVCache.attention on both sides of the rule, against the oracle."""
+    c = case(12, 14, 2, 64, 16, dtype, qlens, cached)
+    want = ref.attention(c["q"], c["pool"], c["slices"], c["tables"], c["ctx"], 14, 2)
+    cache = PagedKVCache(1, c["NB"], 16, 2, 64, DEV, dtype)
+    cache.pools[0].copy_(c["pool"])
+    pos = torch.tensor(c["pos"], device=DEV)
+    got = cache.attention(0, c["q"].to(DEV), pos, c["slices"], c["tables"], c["ctx"])
+    meta = cache.step_metadata(pos, c["slices"], c["tables"], c["ctx"], cache.rows_per_item(14), num_heads=14)
+    assert bool(meta.num_columns_work) == columns
     torch.testing.assert_close(got.cpu().float(), want.float(),
                                **(dict(atol=1e-5, rtol=0) if dtype == torch.float32 else TOL))

@@ -9,7 +9,7 @@ import pytest
 
 from tinybatch_amd.kv_cache import PagedKVCache
 from tinybatch_amd.metadata import (TILE_PARTITION, ColumnsRoute, PrefillRoute, build_columns_work,
-                                    build_step_metadata, columns_partition)
+                                    build_step_metadata, columns_partition, columns_pay)
 
 
 def covered(first, pos0, rows, hq, hkv, work, part):
@@ -102,3 +102,34 @@ def test_partition_of_very_long_prompts():
     t = time.perf_counter()
     assert columns_partition([0], [1 << 23], r) % 64 == 0
     assert time.perf_counter() - t < 0.3
+
+
+@pytest.mark.parametrize("hq,hkv,d,dtype,prompts,others,want", [
+    (14, 2, 64, 2, [(0, 40)], 4, False),              # tiles beside decode rows: one launch
+    (14, 2, 64, 2, [(0, 700)], 4, False),
+    (14, 2, 64, 2, [(0, 1500)] * 4, 4, True),
+    (14, 2, 64, 2, [(8000, 300)], 4, True),           # as work items otherwise
+    (14, 2, 64, 2, [(0, 700)] * 4, 0, False),
+    (14, 2, 64, 2, [(0, 700)] * 16, 0, True),
+    (14, 2, 64, 1, [(3000, 100)] * 12, 0, True),
+    (8, 8, 64, 2, [(0, 850)] * 16, 0, False),         # one head per kv head
+    (32, 8, 128, 2, [(0, 280)], 0, True),
+    (32, 8, 128, 2, [(0, 40)], 4, False),
+    (14, 2, 64, 0, [(0, 16)], 0, False),
+    (14, 2, 64, 0, [(0, 100)] * 16, 0, True),
+    (14, 2, 64, 0, [(1008, 16)], 8, False),
+    (32, 8, 128, 0, [(0, 400)], 0, True),
+    (14, 2, 64, 2, [], 4, False)])
+def test_where_the_column_tiles_pay(hq, hkv, d, dtype, prompts, others, want):
+    """Either side of the rule's lines, as both routes measured."""
+    seqs = [(c, n) for c, n in prompts] + [(500, 1)] * others
+    ends = np.cumsum([n for _, n in seqs]).tolist()
+    slices = list(zip([0] + ends[:-1], ends))
+    assert columns_pay(slices, [c + n for c, n in seqs], ColumnsRoute(hq, hkv, d, 8, 256, dtype), dtype != 0) == want
+
+
+def test_rule_refuses_what_the_work_list_refuses():
+    with pytest.raises(RuntimeError):
+        columns_pay([(0, 16)], [100], ColumnsRoute(14, 4, 64, 8, 256), True)
+    with pytest.raises(RuntimeError):
+        columns_pay([(0, 16)], [100], ColumnsRoute(14, 2, 96, 8, 256), True)

@@ -106,6 +106,7 @@ SIGNATURES = {
         c_vp, c_sz,                              # workspace, bytes
         c_vp, c_vp, c_i32, c_vp]),               # rope cos, sin, max position, stream
     "tb_prefill_columns_partition": (c_i32, [c_vp, c_vp, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32]),
+    "tb_prefill_columns_pay": (c_i32, [c_vp, c_vp, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32]),
     "tb_build_prefill_columns_work": (c_i32, [c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32,
                                               c_vp, c_i32, c_vp]),
     "tb_prefill_stream_max_context": (c_i32, [c_i32]),

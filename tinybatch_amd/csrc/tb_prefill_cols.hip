@@ -684,54 +684,190 @@ struct column_tiles {
 
 }  // namespace
 
+namespace {
+
+// What a step of column tiles costs, in us: a workgroup alone on its CU takes 1.0 (head
+// dim 64) or 1.6 us a chunk, a full CU 0.65 or 1.05 us per chunk of its workgroups (fp32, at
+// the matrix rate either way: 4 or 8 and 3.6 or 7.2, to the proportion that counts here: with
+// the sums in short chains they measure 1.5 times that); a split
+// adds the merge's launch (5 us) and its rows' partials, written and read (4 bytes/ps).
+struct columns_price {
+  const column_tiles& tiles;
+  bool f32;
+  int hkv;
+  double alone, full, share, slot_bytes;
+
+  columns_price(const column_tiles& t, int num_heads, int num_kv_heads, int head_dim, int32_t dtype, int num_cus)
+      : tiles(t), f32(dtype == TB_DTYPE_F32), hkv(num_kv_heads) {
+    const bool d64 = head_dim == 64;
+    alone = f32 ? (d64 ? 4.0 : 8.0) : d64 ? 1.0 : 1.6;
+    full = f32 ? (d64 ? 3.6 : 7.2) : d64 ? 0.65 : 1.05;
+    share = full * (double)(tiles.chunks * hkv) / num_cus;
+    slot_bytes = (double)num_heads * (head_dim + 2) * 4;
+  }
+  double one(int chunks) const {   // us a chunk takes the longest workgroup
+    const bool two_sets = !f32 && tiles.entries(chunks) * hkv <= COLS_SHARED;
+    return two_sets ? 0.66 * alone : alone;
+  }
+  // rows unsplit (chunks == tiles.longest) or in parts of `chunks`, without the merge
+  double span(int chunks) const { return std::max(one(chunks) * chunks, share + 0.5 * full * chunks); }
+  // the merge of rows in parts of `chunks`, of which `partials` are written and read: it reads
+  // eight partials at a time, and each eight more are another round trip
+  double merge(int chunks, int64_t partials) const {
+    return 5.0 + 3.0 * ((tiles.longest - 1) / chunks / 8) + 2 * partials * slot_bytes / 4e6;
+  }
+};
+
+// The partitions of a step's rows in parts of `tokens` positions: of split rows, of all rows.
+void count_partitions(const int32_t* pos0, const int32_t* new_rows, int num_seqs, int64_t tokens, int64_t* split,
+                      int64_t* all) {
+  *split = *all = 0;
+  for (int i = 0; i < num_seqs; ++i) {
+    // rows of k partitions: positions (k - 1) tokens .. k tokens - 1
+    const int64_t first = pos0[i], last = first + new_rows[i];
+    for (int64_t k = first / tokens + 1; (k - 1) * tokens < last; ++k) {
+      const int64_t rows_k = std::min(last, k * tokens) - std::max(first, (k - 1) * tokens);
+      *all += k * rows_k;
+      if (k > 1) *split += k * rows_k;
+    }
+  }
+}
+
+// The partition of least cost in chunks (past the longest context: no row is split). Measured
+// in a graph with the append, bf16, 14 / 2 heads of 64, us per layer: 16 prefix hits
+// of 100 rows after 3008 positions 41.4 (45.4 when split at 512 positions), 4 of 30 after
+// 704 14.2 (16.9), one fresh prompt of 600 unsplit 16.8 (17.7).
+int best_partition(const columns_price& price, const int32_t* pos0, const int32_t* new_rows, int num_seqs,
+                   int64_t other_partitions) {
+  const int longest = price.tiles.longest;
+  int best = longest + 1;
+  double cost = price.span(longest);
+  for (int part = 4; part < longest; part += part < 16 ? 2 : part < 64 ? 8 : 32) {
+    int64_t split, all;
+    count_partitions(pos0, new_rows, num_seqs, (int64_t)part * CHUNK, &split, &all);
+    // a call without a workspace still finds room: shorter than the tiles' 1024 positions only
+    // while the step's partials fit the static scratch
+    if (part < 16 && (all + other_partitions) * price.slot_bytes > TB_NOALLOC_SCRATCH_BYTES) continue;
+    const double c = price.span(part) + price.merge(part, split);
+    if (c < 0.95 * cost) cost = c, best = part;
+  }
+  return best;
+}
+
+bool columns_shape_ok(int32_t head_dim, int32_t dtype) {
+  return (head_dim == 64 || head_dim == 128) &&
+         (dtype == TB_DTYPE_F32 || dtype == TB_DTYPE_F16 || dtype == TB_DTYPE_BF16);
+}
+
+}  // namespace
+
 extern "C" int32_t tb_prefill_columns_partition(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs,
                                                 int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
                                                 int32_t dtype, int32_t num_cus, int32_t other_partitions) {
   if (!columns_args_ok(pos0, new_rows, num_seqs, num_heads, num_kv_heads) || num_cus <= 0 || other_partitions < 0)
     return TB_ERR_INVALID_ARG;
-  if ((head_dim != 64 && head_dim != 128) || (dtype != TB_DTYPE_F32 && dtype != TB_DTYPE_F16 && dtype != TB_DTYPE_BF16))
-    return TB_ERR_INVALID_ARG;
+  if (!columns_shape_ok(head_dim, dtype)) return TB_ERR_INVALID_ARG;
+  const column_tiles tiles(pos0, new_rows, num_seqs, num_heads / num_kv_heads);
+  const columns_price price(tiles, num_heads, num_kv_heads, head_dim, dtype, num_cus);
+  return best_partition(price, pos0, new_rows, num_seqs, other_partitions) * CHUNK;
+}
+
+// The two routes priced, in us without the launch and append they share. Fitted to times in a
+// graph of both routes for 1128 steps (1 to 16 prompts of 16 to 4000 rows after 0 to 8000
+// positions, alone and beside 4 to 40 decode rows, 1 to 8 heads per kv head, head dims 64 and
+// 128); the route taken is then within 5% of the better one for 97% of them. What it comes to,
+// us per layer with the append:
+// - beside other rows the column tiles are a launch of their own, where tiles and work items
+//   share one: bf16, 14 / 2 heads of 64, 4 decode rows: a prompt of 40 18.5 (tiles 11.5), of 3000
+//   50.1 (49.6), 4 of 1500 43.5 (51.6), 8 of 1500 70.6 (95.8);
+// - at head dim 64, fresh prompts the tiles take whole (1024 positions): 4 of 700 20.3
+//   (19.2), 16 of 700 40.7 (43.8); with one head per kv head 16 of 850 56.8 (51.4);
+// - fp32: prompts of 16 to 200 rows 11.8..30.7 (work items 8.5..15.7), 16 of 100 21 (31).
+extern "C" int32_t tb_prefill_columns_pay(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs,
+                                          int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t dtype,
+                                          int32_t num_cus, int32_t tiles_served, int32_t beside_others) {
+  if (!columns_args_ok(pos0, new_rows, num_seqs, num_heads, num_kv_heads) || num_cus <= 0) return TB_ERR_INVALID_ARG;
+  if (!columns_shape_ok(head_dim, dtype)) return TB_ERR_INVALID_ARG;
+  if (num_seqs == 0) return 0;
+  const bool d64 = head_dim == 64, f32 = dtype == TB_DTYPE_F32;
   const int rep = num_heads / num_kv_heads;
   const column_tiles tiles(pos0, new_rows, num_seqs, rep);
-  const int longest = tiles.longest;
-  // The partition with the least cost, in us: a workgroup alone on its CU takes 1.0 (head
-  // dim 64) or 1.6 us a chunk, a full CU 0.65 or 1.05 us per chunk of its workgroups (fp32, at
-  // the matrix rate either way: 4 or 8 and 3.6 or 7.2); a split
-  // adds the merge's launch (5 us) and its rows' partials, written and read (4 bytes/ps).
-  // Measured in a graph with the append, bf16, 14 / 2 heads of 64, us per layer: 16 prefix hits
-  // of 100 rows after 3008 positions 41.4 (45.4 when split at 512 positions), 4 of 30 after
-  // 704 14.2 (16.9), one fresh prompt of 600 unsplit 16.8 (17.7).
-  const bool d64 = head_dim == 64, f32 = dtype == TB_DTYPE_F32;
-  const double alone = f32 ? (d64 ? 4.0 : 8.0) : d64 ? 1.0 : 1.6, full = f32 ? (d64 ? 3.6 : 7.2) : d64 ? 0.65 : 1.05;
-  const double share = full * (double)(tiles.chunks * num_kv_heads) / num_cus;
-  auto span = [&](int chunks) {
-    const int64_t wgs = tiles.entries(chunks) * num_kv_heads;
-    const double one = !f32 && wgs <= COLS_SHARED ? 0.66 * alone : alone;   // two sets of waves on its chunks
-    return std::max(one * chunks, share + 0.5 * full * chunks);
-  };
-  int best = longest + 1;                              // longer than every context: no row is split
-  double cost = span(longest);
-  for (int part = 4; part < longest; part += part < 16 ? 2 : part < 64 ? 8 : 32) {
-    const int64_t tokens = (int64_t)part * CHUNK;
-    int64_t parts = 0, slots = other_partitions;       // partials of split rows; partitions of all rows
-    for (int i = 0; i < num_seqs; ++i) {
-      // rows of k partitions: positions (k - 1) tokens .. k tokens - 1
-      const int64_t first = pos0[i], last = first + new_rows[i];
-      for (int64_t k = first / tokens + 1; (k - 1) * tokens < last; ++k) {
-        const int64_t rows_k = std::min(last, k * tokens) - std::max(first, (k - 1) * tokens);
-        slots += k * rows_k;
-        if (k > 1) parts += k * rows_k;
+  const columns_price price(tiles, num_heads, num_kv_heads, head_dim, dtype, num_cus);
+  const int part = best_partition(price, pos0, new_rows, num_seqs, 0), chunks = std::min(part, tiles.longest);
+  const bool split = part <= tiles.longest;
+  int64_t split_parts = 0, all_parts = 0;
+  if (split) count_partitions(pos0, new_rows, num_seqs, (int64_t)part * CHUNK, &split_parts, &all_parts);
+  double columns = split ? price.merge(part, split_parts) : 0.0;
+  // a launch of its own, while the merge is there anyway (fp32: the others' chain is the longer one)
+  if (beside_others) columns += !split ? 6.0 : !f32 ? 1.0 : d64 ? 5.0 : 8.0;
+  double other = 0.0;
+  if (f32) {
+    // in the kernel's own chunks of 32, by the waves that have columns
+    int64_t longest_half = 0, busy = 0;
+    for (int i = 0; i < num_seqs; ++i)
+      for (int c = 0; c < new_rows[i] * rep; c += COLS) {
+        const int64_t n = (columns_limit(pos0[i], new_rows[i], rep, c) + 31) / 32;
+        longest_half = std::max(longest_half, n);
+        busy += n * ((std::min(COLS, new_rows[i] * rep - c) + 31) / 32);
       }
+    columns += 1.0 + std::max((d64 ? 3.1 : 5.3) * (split ? 2 * chunks : longest_half),
+                              (d64 ? 2.9 : 6.0) * (0.25 * busy * num_kv_heads / num_cus + chunks));
+    int64_t longest_ctx = 0, items = 0, reads = 0, kv = 0;   // work items, positions they read, the pool's positions
+    for (int i = 0; i < num_seqs; ++i) {
+      const int64_t n = new_rows[i], c = (int64_t)pos0[i] + n;
+      longest_ctx = std::max(longest_ctx, c);
+      items += n * ((c + 255) / 256);
+      reads += n * pos0[i] + n * (n + 1) / 2;
+      kv += c;
     }
-    const double slot_bytes = (double)num_heads * (head_dim + 2) * 4;
-    // a call without a workspace still finds room: shorter than the tiles' 1024 positions only
-    // while the step's partials fit the static scratch
-    if (part < 16 && slots * slot_bytes > TB_NOALLOC_SCRATCH_BYTES) continue;
-    // the merge reads eight partials at a time: each eight more are another round trip
-    const double c = span(part) + 5.0 + 3.0 * ((longest - 1) / part / 8) + 2 * parts * slot_bytes / 4e6;
-    if (c < 0.95 * cost) cost = c, best = part;
+    int group = d64 ? 14 : 15;                         // heads per workgroup (tb_paged_attention)
+    while (rep % group) --group;
+    const double wgs = (double)items * num_kv_heads * (rep / group), kr = 1e-3 * reads * num_kv_heads * (rep / group);
+    const bool brief = longest_ctx <= 64 && !beside_others;
+    if (group <= (brief ? 8 : 5) && wgs >= (brief ? 128 : 320) * group) {   // the VALU kernel
+      const double chain = (9.0 + 4.0 * group) * (beside_others ? 1.0 : std::min<int64_t>(longest_ctx, 256) / 256.0);
+      other = (d64 ? 1.0 : 2.0) * (0.6 * chain + 0.00025 * (1 + group) * wgs + (0.0058 + 0.0087 * group) * kr) +
+              0.35e-3 * std::max(0.0, (double)kv * num_kv_heads - (d64 ? 50e3 : 25e3));   // K/V past the L2s
+    } else {
+      other = d64 ? 0.0045 * wgs + 0.058 * kr : 0.0055 * wgs + 0.12 * kr;
+    }
+    if (longest_ctx > 256 && !beside_others) other += 5.0;
+    return columns < 0.92 * other;
   }
-  return best * CHUNK;
+  // columns: a workgroup's rows cross the diagonal over rows / 64 chunks, of which its waves
+  // use a part
+  const double cross = 2.0 * COLS / rep / 64;
+  const double share = price.share + price.full * cross * (double)tiles.entries(tiles.longest) * num_kv_heads / num_cus;
+  columns += 2.0 + std::max(price.one(part) * (chunks + cross), share + 0.5 * price.full * chunks);
+  // 64-row tiles of one head in parts of 1024 positions; longer tails as work items
+  int group = 16;
+  while (rep % group) --group;
+  const int rows_per_item = std::max(1, 16 / group);
+  int64_t tile_chunks = 0, items = 0, partials = 0;
+  int longest = 0;
+  bool merge = false;
+  for (int i = 0; i < num_seqs; ++i) {
+    const int64_t n = new_rows[i], c = (int64_t)pos0[i] + n;
+    if (!tiles_served || (c > 4096 && c > 16 * n)) {   // metadata.tiles_sequence
+      items += (n + rows_per_item - 1) / rows_per_item * ((c + 255) / 256) * num_kv_heads * (rep / group);
+      partials += n * ((c + 255) / 256);
+      merge |= c > 256;
+      continue;
+    }
+    for (int64_t r = 0; r < n; r += 64) {
+      const int64_t end = pos0[i] + std::min<int64_t>(n, r + 64), whole = end / 1024, rest = end % 1024;
+      tile_chunks += whole * 16 + (rest + 63) / 64;
+      longest = std::max(longest, whole ? 16 : (int)((rest + 63) / 64));
+      if (end > 1024) partials += 64 * ((end + 1023) / 1024), merge = true;
+    }
+  }
+  const double tile_alone = d64 ? 0.82 : 3.1, tile_full = d64 ? 0.61 : 1.6;
+  const double tile_share = tile_full * (double)(tile_chunks * num_heads) / num_cus;
+  if (longest > 0)
+    other += std::max(tile_alone * longest + (d64 ? 0.3 : 0.75) * tile_share, tile_share + 0.3 * tile_full * longest);
+  other += (d64 ? 0.0135 : 0.028) * items + partials * price.slot_bytes / 4e6;
+  if (merge && !beside_others) other += 5.0;
+  return columns < 0.97 * other;
 }
 
 extern "C" int32_t tb_build_prefill_columns_work(const int32_t* first_row, const int32_t* seq_index, const int32_t* pos0,

@@ -29,7 +29,7 @@ import numpy as np
 import torch
 
 from . import _lib, ops
-from .metadata import StepMetadata, build_step_metadata
+from .metadata import StepMetadata, build_step_metadata, columns_pay
 
 
 class PagedKVCache:
@@ -73,7 +73,8 @@ class PagedKVCache:
         beside a run of decode rows to tb_paged_prefill and the decode kernel, each
         on its own rows (ops.attach_split_parts), when the decode rows gain by it. In any
         other step (longer contexts, fp32) sequences of >= 16 new rows go to
-        tb_paged_prefill_columns (ops.columns_route).
+        tb_paged_prefill_columns (ops.columns_route) where that is the faster one
+        (metadata.columns_pay), and to tiles (16-bit) or work items otherwise.
         """
         pos_key = (positions, positions._version) if isinstance(positions, torch.Tensor) else list(positions)
         for e in self._meta_cache:
@@ -87,7 +88,7 @@ class PagedKVCache:
         # 16-bit pools serve long runs of new rows (prefills) with the tile kernel; a
         # step of prefills only (every sequence >= 16 new rows, its context within
         # the kernel's limit) goes to tb_paged_prefill instead; in other steps such runs go
-        # to the column tiles, decode rows and short tails to the work items beside them
+        # to the column tiles where they pay for a launch of their own
         tile = self.pools[0].dtype in (torch.float16, torch.bfloat16)
         route = None
         if num_heads is not None and context_lens is not None and self.device.type == "cuda" and tile:
@@ -100,6 +101,8 @@ class PagedKVCache:
         if num_heads is not None and context_lens is not None and self.device.type == "cuda" and route is None:
             columns = ops.columns_route(self.dtype, num_heads, self.n_kv_heads, self.head_dim, self.block_size,
                                         self.device)
+            if columns is not None and not columns_pay(seq_slices, context_lens, columns, tile):
+                columns = None                            # tiles and work items, in one launch
         meta = build_step_metadata(positions if host_positions is None else host_positions,
                                    seq_slices, block_tables, context_lens,
                                    block_size=self.block_size, num_blocks=self.num_blocks,

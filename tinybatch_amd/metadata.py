@@ -297,6 +297,24 @@ def columns_partition(pos0s, new_rows, route: ColumnsRoute, other_partitions: in
     return p
 
 
+def columns_pay(seq_slices, context_lens, route: ColumnsRoute, tiles: bool) -> bool:
+    """tb_prefill_columns_pay: whether the column tiles serve the step's sequences of >= 16 new
+    rows faster than the tiles (``tiles``: 16-bit steps have them) and work items."""
+    from . import _lib
+
+    n = [int(e) - int(b) for b, e in seq_slices]
+    seqs = [(int(c) - q, q) for q, c in zip(n, context_lens) if q >= 16]
+    if not seqs or any(p < 0 for p, _ in seqs):           # the builder refuses the latter
+        return False
+    a, ptrs = _column_arrays(*[[x[0] for x in seqs]] * 3, [x[1] for x in seqs])
+    r = int(_lib.lib().tb_prefill_columns_pay(ptrs[2], ptrs[3], a.shape[1], route.num_heads, route.num_kv_heads,
+                                              route.head_dim, route.dtype, route.num_cus, int(tiles),
+                                              int(any(0 < q < 16 for q in n))))
+    if r < 0:
+        _lib.check(r, "tb_prefill_columns_pay")
+    return r == 1
+
+
 def build_columns_work(first_rows, seqs, pos0s, new_rows, partition: int, route: ColumnsRoute) -> np.ndarray:
     """tb_build_prefill_columns_work: int32 [n, 8], entry g for XCD g % route.num_xcds."""
     import ctypes
