@@ -37,6 +37,7 @@
 // chunk's loads spread between its products (the same); row sums on the matrix unit (5%
 // slower at head dim 64).
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <vector>
 
@@ -634,7 +635,6 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void paged_prefill_columns_f3
 namespace {
 
 constexpr int COLS = tb::cshape<64>::COLS, CHUNK = tb::cshape<64>::CK;
-constexpr int COLS_SHARED = 256;   // workgroups up to which two sets of waves share one's chunks
 static_assert(COLS == tb::cshape<128>::COLS && CHUNK == tb::cshape<128>::CK, "one work list for both head dims");
 
 struct col_entry {
@@ -694,11 +694,11 @@ namespace {
 struct columns_price {
   const column_tiles& tiles;
   bool f32;
-  int hkv;
+  int hkv, cus;
   double alone, full, share, slot_bytes;
 
   columns_price(const column_tiles& t, int num_heads, int num_kv_heads, int head_dim, int32_t dtype, int num_cus)
-      : tiles(t), f32(dtype == TB_DTYPE_F32), hkv(num_kv_heads) {
+      : tiles(t), f32(dtype == TB_DTYPE_F32), hkv(num_kv_heads), cus(num_cus) {
     const bool d64 = head_dim == 64;
     alone = f32 ? (d64 ? 4.0 : 8.0) : d64 ? 1.0 : 1.6;
     full = f32 ? (d64 ? 3.6 : 7.2) : d64 ? 0.65 : 1.05;
@@ -706,7 +706,7 @@ struct columns_price {
     slot_bytes = (double)num_heads * (head_dim + 2) * 4;
   }
   double one(int chunks) const {   // us a chunk takes the longest workgroup
-    const bool two_sets = !f32 && tiles.entries(chunks) * hkv <= COLS_SHARED;
+    const bool two_sets = !f32 && tiles.entries(chunks) * hkv <= cus;   // as launch_columns
     return two_sets ? 0.66 * alone : alone;
   }
   // rows unsplit (chunks == tiles.longest) or in parts of `chunks`, without the merge
@@ -940,15 +940,27 @@ extern "C" int32_t tb_build_prefill_columns_work(const int32_t* first_row, const
 
 namespace {
 
-// At most one workgroup per CU (256): two sets of waves share its chunks, which then take
+// The CUs of the current device (asked once; 256 where that fails).
+int device_cus() {
+  constexpr int MAX_DEVICES = 64;
+  static std::atomic<int> cus[MAX_DEVICES];
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return 256;
+  if ((n = cus[dev].load(std::memory_order_relaxed)) > 0) return n;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+  cus[dev].store(n, std::memory_order_relaxed);
+  return n;
+}
+
+// At most one workgroup per CU: two sets of waves share its chunks, which then take
 // 0.66 us each instead of 1.0 (head dim 64). Twelve prefix hits of 40..400 rows after
 // 600..3600 positions, 4 fp16 layers with the append: 149 us unsplit against 162 for one set
-// of waves and rows split at 896 positions. Past 256 workgroups one set each leaves room
+// of waves and rows split at 896 positions. Past one per CU (256) one set each leaves room
 // for a second workgroup on the CU, whose start and end then overlap.
 template <typename Tag, int D>
 void launch_columns(const tb::cols_args& a, int num_work, hipStream_t stream) {
   constexpr int T = 64 * tb::cshape<D>::NW;
-  if (num_work <= COLS_SHARED)
+  if (num_work <= device_cus())
     hipLaunchKernelGGL((tb::paged_prefill_columns_kernel<Tag, D, 2>), dim3(num_work), dim3(2 * T), 0, stream, a);
   else
     hipLaunchKernelGGL((tb::paged_prefill_columns_kernel<Tag, D, 1>), dim3(num_work), dim3(T), 0, stream, a);
