@@ -2,6 +2,9 @@
 sequence's rows may see is covered by exactly one entry; padding entries have no rows; the
 partition rule keeps rows whole when the step fills the GPU and never asks for more
 scratch than the tiles did, past the static scratch."""
+import os
+import subprocess
+import sys
 import time
 
 import numpy as np
@@ -133,3 +136,22 @@ def test_rule_refuses_what_the_work_list_refuses():
         columns_pay([(0, 16)], [100], ColumnsRoute(14, 4, 64, 8, 256), True)
     with pytest.raises(RuntimeError):
         columns_pay([(0, 16)], [100], ColumnsRoute(14, 2, 96, 8, 256), True)
+
+
+def test_a_list_past_the_memory_is_an_error():
+    """An allocation that fails behind the C entry is a status, not an exception out of it."""
+    code = """
+import ctypes, resource, sys
+lib = ctypes.CDLL(sys.argv[1])
+page = resource.getpagesize() * int(open("/proc/self/statm").read().split()[0])
+resource.setrlimit(resource.RLIMIT_AS, (page + (256 << 20),) * 2)
+one = lambda x: ctypes.byref(ctypes.c_int32(x))
+n = ctypes.c_int32()
+st = lib.tb_build_prefill_columns_work(one(0), one(0), one((1 << 30) - (1 << 20)), one(1 << 20), 1, 1, 1, 64, 8, 256,
+                                       None, 0, ctypes.byref(n))
+print("status", st)
+"""
+    from tinybatch_amd.build import LIB_PATH
+    r = subprocess.run([sys.executable, "-c", code, LIB_PATH], capture_output=True, text=True, timeout=120,
+                       env={**os.environ, "HIP_VISIBLE_DEVICES": ""})
+    assert r.returncode == 0 and r.stdout.startswith("status -"), (r.returncode, r.stdout, r.stderr[-300:])

@@ -39,6 +39,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <exception>
 #include <vector>
 
 #include "tb_stream.h"
@@ -767,9 +768,13 @@ extern "C" int32_t tb_prefill_columns_partition(const int32_t* pos0, const int32
   if (!columns_args_ok(pos0, new_rows, num_seqs, num_heads, num_kv_heads) || num_cus <= 0 || other_partitions < 0)
     return TB_ERR_INVALID_ARG;
   if (!columns_shape_ok(head_dim, dtype)) return TB_ERR_INVALID_ARG;
-  const column_tiles tiles(pos0, new_rows, num_seqs, num_heads / num_kv_heads);
-  const columns_price price(tiles, num_heads, num_kv_heads, head_dim, dtype, num_cus);
-  return best_partition(price, pos0, new_rows, num_seqs, other_partitions) * CHUNK;
+  try {
+    const column_tiles tiles(pos0, new_rows, num_seqs, num_heads / num_kv_heads);
+    const columns_price price(tiles, num_heads, num_kv_heads, head_dim, dtype, num_cus);
+    return best_partition(price, pos0, new_rows, num_seqs, other_partitions) * CHUNK;
+  } catch (const std::exception&) {   // no memory for a step of this size
+    return TB_ERR_INVALID_ARG;
+  }
 }
 
 // The two routes priced, in us without the launch and append they share. Fitted to times in a
@@ -783,9 +788,9 @@ extern "C" int32_t tb_prefill_columns_partition(const int32_t* pos0, const int32
 // - at head dim 64, fresh prompts the tiles take whole (1024 positions): 4 of 700 20.3
 //   (19.2), 16 of 700 40.7 (43.8); with one head per kv head 16 of 850 56.8 (51.4);
 // - fp32: prompts of 16 to 200 rows 11.8..30.7 (work items 8.5..15.7), 16 of 100 21 (31).
-extern "C" int32_t tb_prefill_columns_pay(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs,
-                                          int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t dtype,
-                                          int32_t num_cus, int32_t tiles_served, int32_t beside_others) {
+static int32_t columns_pay(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs, int32_t num_heads,
+                           int32_t num_kv_heads, int32_t head_dim, int32_t dtype, int32_t num_cus,
+                           int32_t tiles_served, int32_t beside_others) {
   if (!columns_args_ok(pos0, new_rows, num_seqs, num_heads, num_kv_heads) || num_cus <= 0) return TB_ERR_INVALID_ARG;
   if (!columns_shape_ok(head_dim, dtype)) return TB_ERR_INVALID_ARG;
   if (num_seqs == 0) return 0;
@@ -870,10 +875,21 @@ extern "C" int32_t tb_prefill_columns_pay(const int32_t* pos0, const int32_t* ne
   return columns < 0.97 * other;
 }
 
-extern "C" int32_t tb_build_prefill_columns_work(const int32_t* first_row, const int32_t* seq_index, const int32_t* pos0,
-                                                 const int32_t* new_rows, int32_t num_seqs, int32_t num_heads,
-                                                 int32_t num_kv_heads, int32_t partition_tokens, int32_t num_xcds,
-                                                 int32_t num_cus, int32_t* work, int32_t capacity, int32_t* count) {
+extern "C" int32_t tb_prefill_columns_pay(const int32_t* pos0, const int32_t* new_rows, int32_t num_seqs,
+                                          int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, int32_t dtype,
+                                          int32_t num_cus, int32_t tiles_served, int32_t beside_others) {
+  try {
+    return columns_pay(pos0, new_rows, num_seqs, num_heads, num_kv_heads, head_dim, dtype, num_cus, tiles_served,
+                       beside_others);
+  } catch (const std::exception&) {
+    return TB_ERR_INVALID_ARG;
+  }
+}
+
+static int32_t build_columns_work(const int32_t* first_row, const int32_t* seq_index, const int32_t* pos0,
+                                  const int32_t* new_rows, int32_t num_seqs, int32_t num_heads, int32_t num_kv_heads,
+                                  int32_t partition_tokens, int32_t num_xcds, int32_t num_cus, int32_t* work,
+                                  int32_t capacity, int32_t* count) {
   if (!columns_args_ok(pos0, new_rows, num_seqs, num_heads, num_kv_heads) || !count || num_xcds <= 0 || num_cus <= 0)
     return TB_ERR_INVALID_ARG;
   if (num_seqs > 0 && (!first_row || !seq_index)) return TB_ERR_INVALID_ARG;
@@ -936,6 +952,18 @@ extern "C" int32_t tb_build_prefill_columns_work(const int32_t* first_row, const
       w[7] = pc;
     }
   return TB_OK;
+}
+
+extern "C" int32_t tb_build_prefill_columns_work(const int32_t* first_row, const int32_t* seq_index, const int32_t* pos0,
+                                                 const int32_t* new_rows, int32_t num_seqs, int32_t num_heads,
+                                                 int32_t num_kv_heads, int32_t partition_tokens, int32_t num_xcds,
+                                                 int32_t num_cus, int32_t* work, int32_t capacity, int32_t* count) {
+  try {
+    return build_columns_work(first_row, seq_index, pos0, new_rows, num_seqs, num_heads, num_kv_heads,
+                              partition_tokens, num_xcds, num_cus, work, capacity, count);
+  } catch (const std::exception&) {
+    return TB_ERR_INVALID_ARG;
+  }
 }
 
 namespace {
