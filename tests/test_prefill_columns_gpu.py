@@ -13,7 +13,7 @@ import torch
 from oracle import reference_path as ref
 from test_prefill_columns_work import both_routes
 from test_prefill_stream_gpu import DEV, TOL, case
-from tinybatch_amd import layer_ops, ops
+from tinybatch_amd import layer_ops, metadata as step_metadata, ops
 from tinybatch_amd.kv_cache import PagedKVCache
 from tinybatch_amd.metadata import TILE_PARTITION, build_step_metadata
 from tinybatch_amd.model import rope_tables
@@ -54,8 +54,8 @@ def test_edges_of_tiles_and_chunks(Hq, Hkv, D, dtype):
 
 
 @pytest.mark.parametrize("BS", [16, 32, 64])
-def test_more_chunks_than_one_read_of_block_ids(BS):
-    # 4097 .. 4300 positions: chunks 64 .. 67; few rows, so the rows are split as well
+def test_long_contexts_of_few_rows(BS):
+    # 4097 .. 4300 positions: few rows, so that they are split
     meta = check(case(2, 14, 2, 64, BS, torch.bfloat16, [16, 40], [4081, 4260]))
     assert meta.num_split_rows == 56
     check(case(3, 2, 1, 64, BS, torch.float16, [4200], [0]))
@@ -170,3 +170,87 @@ def test_cache_takes_the_faster_route(dtype, qlens, cached, columns):
     assert bool(meta.num_columns_work) == columns
     torch.testing.assert_close(got.cpu().float(), want.float(),
                                **(dict(atol=1e-5, rtol=0) if dtype == torch.float32 else TOL))
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,dtype,qlens,cached,sets", [
+    (14, 2, 64, torch.bfloat16, [16, 40], [4081, 8300], 2), (14, 2, 64, torch.float16, [16, 40], [4081, 8300], 2),
+    (32, 8, 128, torch.float16, [33, 16], [8500, 4200], 2),
+    (8, 8, 64, torch.bfloat16, [4250], [0], 1), (32, 8, 128, torch.bfloat16, [1100], [4300], 1),
+    (14, 2, 64, torch.float32, [30, 18], [2100, 6300], 1), (32, 8, 128, torch.float32, [33], [4200], 1)])
+def test_block_ids_of_a_part_past_the_first_64_chunks(Hq, Hkv, D, dtype, qlens, cached, sets, monkeypatch):
+    """Rows kept whole, so that a workgroup walks more than 64 chunks (fp32: of 32 positions) and
+    reads block ids again; with one set of waves, and with two (up to 256 entries)."""
+    monkeypatch.setattr(step_metadata, "columns_partition", lambda *a: 1 << 20)
+    c = case(15, Hq, Hkv, D, 16, dtype, qlens, cached)
+    meta = check(c)
+    longest = max(c["ctx"])
+    assert meta.num_split_rows == 0 and -(-longest // (32 if dtype == torch.float32 else 64)) > 65
+    assert dtype == torch.float32 or (meta.num_columns_work <= 256) == (sets == 2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("cached,part", [(0, 1 << 20), (300, 512)])
+def test_one_set_of_waves_at_head_dim_128(dtype, cached, part, monkeypatch):
+    """More than 256 entries, rows whole and split, an odd last tile."""
+    monkeypatch.setattr(step_metadata, "columns_partition", lambda *a: part)
+    meta = check(case(16, 32, 8, 128, 16, dtype, [1237], [cached]))
+    assert meta.num_columns_work > 256 and (meta.num_split_rows > 0) == (part == 512)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(14, 2, 64), (32, 8, 128)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("log2_p,n,whole", [(14, 40, False), (16, 40, True), (16, 600, True), (18, 600, True),
+                                            (22, 600, False)])
+def test_one_dominant_key(Hq, Hkv, D, dtype, log2_p, n, whole, monkeypatch):
+    """One key of weight 1 and 3999 of 2^-14 .. 2^-22, from 2^-15 on subnormal in fp16: the products
+    with their values (ones beside a zero) and the row sum count them alike (a sum that dropped
+    them would be 6% off at 2^-16). Bound: all weights are rounded the same way, by up to half a
+    unit of 2^-24 in fp16, and the outputs by 2^-9 in bf16."""
+    if whole:
+        monkeypatch.setattr(step_metadata, "columns_partition", lambda *a: 1 << 20)
+    bound = 2.0 ** (log2_p - 25) + 2.0 ** -8
+    ctx = 4000
+    k = torch.full((ctx, Hkv, D), 0.0)
+    k[1:, :, 0] = -log2_p * 0.6931471805599453 / 8
+    v = torch.ones(ctx, Hkv, D)
+    v[0] = 0
+    q = torch.zeros(n, Hq, D)
+    q[:, :, 0] = 8 * D ** 0.5
+    pool = torch.stack([k, v]).reshape(2, ctx // 16, 16, Hkv, D).permute(1, 0, 3, 2, 4).contiguous().to(dtype)
+    route = ops.columns_route(dtype, Hq, Hkv, D, 16, DEV)
+    meta = build_step_metadata(list(range(ctx - n, ctx)), [(0, n)], [list(range(ctx // 16))], [ctx], block_size=16,
+                               num_blocks=ctx // 16, partition_tokens=256, columns_route=route).to(DEV)
+    got = ops.paged_attention(q.to(DEV, dtype), pool.to(DEV), meta, num_heads=Hq).cpu().double().view(n, Hq, D)
+    score = (k[:, 0, 0].to(dtype).double() * q[0, 0, 0].to(dtype).double() * D ** -0.5)
+    weights = torch.exp(score - score[0])
+    for row in (0, n // 2, n - 1):
+        w = weights[1:ctx - n + row + 1].sum().item()
+        assert ((got[row] * (1 + w) / w - 1).abs() <= bound).all(), (row, got[row, 0, 0], w / (1 + w))
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,dtype", [(14, 2, 64, torch.bfloat16), (32, 8, 128, torch.float16),
+                                            (14, 2, 64, torch.float32), (32, 8, 128, torch.float32)])
+def test_non_finite_keys_and_values_of_the_context(Hq, Hkv, D, dtype):
+    """A NaN key reaches every row that sees it and no other; 64 positions of -inf scores weigh
+    nothing; a NaN value of the cached context reaches every row, and no other sequence."""
+    c = case(17, Hq, Hkv, D, 16, dtype, [60, 60, 60, 60], [300, 300, 300, 0])
+    c["q"][:, :, 0] = 1.0
+    at = lambda s, p: (c["tables"][s][p // 16], p % 16)
+    b, o = at(0, 330)
+    c["pool"][b, 0, :, o, 1] = float("nan")                 # rows 30 .. 59 of sequence 0 see it
+    for p in range(64, 128):
+        b, o = at(1, p)
+        c["pool"][b, 0, :, o, 0] = float("-inf")
+    b, o = at(2, 200)
+    c["pool"][b, 1, :, o] = float("nan")
+    want = ref.attention(c["q"], c["pool"], c["slices"], c["tables"], c["ctx"], Hq, Hkv)
+    got = ops.paged_attention(c["q"].to(DEV), c["pool"].to(DEV), metadata(c), num_heads=Hq).cpu()
+    assert got[:30].isfinite().all() and got[30:60].isnan().all() and got[120:180].isnan().all()
+    tol = dict(atol=1e-5, rtol=0) if dtype == torch.float32 else TOL
+    clean = {**c, "pool": c["pool"].clone()}
+    b, o = at(0, 330)
+    clean["pool"][b, 0, :, o, 1] = 0.0                      # rows that do not see it: any finite key there
+    first = ref.attention(c["q"][:60], clean["pool"], [(0, 60)], c["tables"][:1], c["ctx"][:1], Hq, Hkv)
+    torch.testing.assert_close(got[:30].float(), first[:30].float(), **tol)
+    for rows in (slice(60, 120), slice(180, 240)):
+        torch.testing.assert_close(got[rows].float(), want[rows].float(), **tol)
