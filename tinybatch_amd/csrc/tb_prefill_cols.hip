@@ -21,7 +21,9 @@
 //   O^T[d][col]  += V^T[d][pos] . P^T[pos][col]   v_mfma_f32_32x32x16, A = V^T (LDS
 //                                                  transpose reads), B = the S^T registers
 // so that each K or V value read from LDS meets 32 columns, and the online softmax state
-// of column l % 32 lives in lanes l and l ^ 32.
+// of column l % 32 lives in lanes l and l ^ 32. A masked score weighs 0, also against what is
+// not finite: an infinite or NaN value of a new row makes the earlier rows of its workgroup NaN
+// (in the reference's masked product all rows of the sequence); a key's reaches none.
 //
 // What bounds it and what it measured (bf16, us per layer, against the 64-row tiles of
 // tb_attention.hip): three prompts of 5300..7333 tokens at 32 / 8 heads of 128: 1090 us =
@@ -57,7 +59,8 @@ struct cmath<f16_t> {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(shalf8_t, a), __builtin_bit_cast(shalf8_t, b), c,
                                                    0, 0, 0);
   }
-  // acc + the two halves of p (times one each)
+  // acc + the two halves of p (times one each); subnormal halves count, as in the products
+  // (measured: thousands of weights of 2^-16 .. 2^-22 beside one of 1)
   static __device__ __forceinline__ float add2(uint32_t p, uint32_t ones, float acc) {
     return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, p), __builtin_bit_cast(half2_t, ones), acc, false);
   }
