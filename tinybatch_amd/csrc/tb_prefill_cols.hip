@@ -126,8 +126,9 @@ struct cshape {
 };
 
 // SP = 2: two sets of NW waves on the same columns, set sp taking chunks sp, sp + 2, ... of
-// the range through a ring of its own; their states merge in LDS at the end.
-template <typename Tag, int D, int SP>
+// the range through a ring of its own; their states merge in LDS at the end. SIGNED: a scale of
+// zero or below, whose sign goes into q (a branch on it in every launch cost 1% of short ones).
+template <typename Tag, int D, int SP, bool SIGNED>
 __global__ __launch_bounds__(64 * cshape<D>::NW * SP, 2) void paged_prefill_columns_kernel(const cols_args a) {
   using S = cshape<D>;
   using M = cmath<Tag>;
@@ -214,7 +215,7 @@ __global__ __launch_bounds__(64 * cshape<D>::NW * SP, 2) void paged_prefill_colu
     for (int s = 0; s < KS / 2; ++s)            // slices s and s + KS/2 pair (dims i and i + D/2)
       rope_pair<scalar_t>(qv[s], qv[s + KS / 2], a.rope.cos + r + 16 * s, a.rope.sin + r + 16 * s);
   }
-  if (a.q_sign != 1.f) {
+  if constexpr (SIGNED) {
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       typename M::vec8_t x = __builtin_bit_cast(typename M::vec8_t, qv[s]);
@@ -988,13 +989,19 @@ int device_cus() {
 // 600..3600 positions, 4 fp16 layers with the append: 149 us unsplit against 162 for one set
 // of waves and rows split at 896 positions. Past one per CU (256) one set each leaves room
 // for a second workgroup on the CU, whose start and end then overlap.
-template <typename Tag, int D>
-void launch_columns(const tb::cols_args& a, int num_work, hipStream_t stream) {
+template <typename Tag, int D, bool SIGNED>
+void launch_columns_sets(const tb::cols_args& a, int num_work, hipStream_t stream) {
   constexpr int T = 64 * tb::cshape<D>::NW;
   if (num_work <= device_cus())
-    hipLaunchKernelGGL((tb::paged_prefill_columns_kernel<Tag, D, 2>), dim3(num_work), dim3(2 * T), 0, stream, a);
+    hipLaunchKernelGGL((tb::paged_prefill_columns_kernel<Tag, D, 2, SIGNED>), dim3(num_work), dim3(2 * T), 0, stream, a);
   else
-    hipLaunchKernelGGL((tb::paged_prefill_columns_kernel<Tag, D, 1>), dim3(num_work), dim3(T), 0, stream, a);
+    hipLaunchKernelGGL((tb::paged_prefill_columns_kernel<Tag, D, 1, SIGNED>), dim3(num_work), dim3(T), 0, stream, a);
+}
+
+template <typename Tag, int D>
+void launch_columns(const tb::cols_args& a, int num_work, hipStream_t stream) {
+  a.q_sign == 1.f ? launch_columns_sets<Tag, D, false>(a, num_work, stream)
+                  : launch_columns_sets<Tag, D, true>(a, num_work, stream);
 }
 
 }  // namespace
