@@ -122,7 +122,8 @@ def test_partition_of_very_long_prompts():
     (14, 2, 64, 0, [(0, 100)] * 16, 0, True),
     (14, 2, 64, 0, [(1008, 16)], 8, False),
     (32, 8, 128, 0, [(0, 400)], 0, True),
-    (14, 2, 64, 2, [], 4, False)])
+    (14, 2, 64, 2, [], 4, False),
+    (14, 2, 64, 2, [((1 << 30) - 10, 16)], 0, False)])   # past the work list's positions
 def test_where_the_column_tiles_pay(hq, hkv, d, dtype, prompts, others, want):
     """Either side of the rule's lines, as both routes measured."""
     seqs = [(c, n) for c, n in prompts] + [(500, 1)] * others

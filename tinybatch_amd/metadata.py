@@ -304,8 +304,9 @@ def columns_pay(seq_slices, context_lens, route: ColumnsRoute, tiles: bool) -> b
 
     n = [int(e) - int(b) for b, e in seq_slices]
     seqs = [(int(c) - q, q) for q, c in zip(n, context_lens) if q >= 16]
-    if not seqs or any(p < 0 for p, _ in seqs):           # the builder refuses the latter
-        return False
+    rep = max(1, route.num_heads // route.num_kv_heads)
+    if not seqs or any(p < 0 or p + q > 1 << 30 or q * rep > 1 << 28 for p, q in seqs):
+        return False                                      # the builder refuses p < 0, the work list the rest
     a, ptrs = _column_arrays(*[[x[0] for x in seqs]] * 3, [x[1] for x in seqs])
     r = int(_lib.lib().tb_prefill_columns_pay(ptrs[2], ptrs[3], a.shape[1], route.num_heads, route.num_kv_heads,
                                               route.head_dim, route.dtype, route.num_cus, int(tiles),
