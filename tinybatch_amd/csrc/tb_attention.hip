@@ -126,11 +126,13 @@ struct f32_shape {
   static constexpr int NW = NW_;           // waves per workgroup
   static constexpr int SPAN = 16 * NW;     // positions in flight
   static constexpr int PITCH = D + 4;      // floats per (wave, head) row of the merge
+  static constexpr int SHORT_CTX = 512;    // PROMPTS: contexts up to which a tile's values are summed in short chains
   // heads whose merge fits 64 KiB beside the waves' (max, sum) pairs: 14 or 15
   static constexpr int max_heads = (65536 / (NW * (int)sizeof(float)) - 32) / PITCH;
 };
 
-template <int D, int NW_>
+// PROMPTS: steps that may hold prompt rows (decode steps come with the fused append).
+template <int D, int NW_, bool PROMPTS>
 __global__ __launch_bounds__(64 * NW_) void paged_attn_f32_kernel(const attn_args a) {
   using S = f32_shape<D, NW_>;
   constexpr int RB = S::RB, KC = S::KC, VC = S::VC, NW = S::NW;
@@ -243,16 +245,35 @@ __global__ __launch_bounds__(64 * NW_) void paged_attn_f32_kernel(const attn_arg
 #pragma unroll
     for (int e = 0; e < 4 * VC; ++e) acc[e] *= alpha;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float p = fast_exp2(s[j] - m_safe);
-      l += p;
-      const bool seen = vpos + j < p1;     // what stands in for a row past the context counts as zeros
+    for (int j = 0; j < 4; ++j) s[j] = fast_exp2(s[j] - m_safe);
+    l += (s[0] + s[1]) + (s[2] + s[3]);
+    auto value = [&](int j, int c, int i) {  // what stands in for a row past the context counts as zeros
+      return vpos + j < p1 ? bits_to_f32(v[j][c].w[i]) : 0.f;
+    };
+    // Prompt rows of short contexts: the tile's own sums in four chains of 4 positions, apart from
+    // the tiles before it (whole workgroup). Their first rows see so few positions that one chain
+    // of 16 is the larger part of their error: prompts of 31..191, distance from 64-bit results
+    // 1.14e-7 against 1.22e-7 (the VALU kernel 1.18e-7). It costs 3% of a short step; decode steps
+    // are at 1.47e-7 (VALU 1.51e-7) without, prompts at head dim 128 at the VALU kernel's error.
+    if (PROMPTS && ctx <= S::SHORT_CTX) {
 #pragma unroll
       for (int c = 0; c < VC; ++c)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          acc[4 * c + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(seen ? bits_to_f32(v[j][c].w[i]) : 0.f, p,
-                                                                acc[4 * c + i], 0, 0, 0);
+        for (int i = 0; i < 4; ++i) {
+          float4_t pv[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            pv[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(value(j, c, i), s[j], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          acc[4 * c + i] += (pv[0] + pv[1]) + (pv[2] + pv[3]);
+        }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int c = 0; c < VC; ++c)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            acc[4 * c + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(value(j, c, i), s[j], acc[4 * c + i], 0, 0, 0);
     }
   }
   l = sum_xor32(sum_xor16(l));
@@ -1323,8 +1344,9 @@ template <int D, int NW>
 static void launch_f32_nw(const attn_args& a, int num_work, hipStream_t stream) {
   using S = f32_shape<D, NW>;
   const size_t lds = (size_t)NW * (a.group * S::PITCH + 32) * sizeof(float);
-  hipLaunchKernelGGL((paged_attn_f32_kernel<D, NW>), dim3(num_work, a.num_kv_heads, a.rep / a.group), dim3(64 * NW), lds,
-                     stream, a);
+  const dim3 grid(num_work, a.num_kv_heads, a.rep / a.group), block(64 * NW);
+  if (a.k_new || D != 64) hipLaunchKernelGGL((paged_attn_f32_kernel<D, NW, false>), grid, block, lds, stream, a);
+  else hipLaunchKernelGGL((paged_attn_f32_kernel<D, NW, D == 64>), grid, block, lds, stream, a);
 }
 
 // A step of few work items is a chain of latencies: a whole partition in flight (16 waves; 8
