@@ -26,16 +26,18 @@
 // (in the reference's masked product all rows of the sequence); a key's reaches none.
 //
 // What bounds it and what it measured (bf16, us per layer, against the 64-row tiles of
-// tb_attention.hip): three prompts of 5300..7333 tokens at 32 / 8 heads of 128: 1090 us =
-// 994 TFLOP/s against 3260 + 290 for the merge of split rows; four of 1746..3738 at 14 / 2
+// tb_attention.hip): three prompts of 5300..7333 tokens at 32 / 8 heads of 128: 1100 us =
+// 985 TFLOP/s once the clock has settled (1150 to 1500 in the first twenty launches after idle)
+// against 3260 + 290 for the merge of split rows; four of 1746..3738 at 14 / 2
 // heads of 64: 86 us = 670 TFLOP/s against 122 + 14. (A plain 8192^3 library product
-// reaches 1232 TFLOP/s on this card.) At head dim 128 a chunk takes a SIMD's two waves
-// 3800 cycles, 2050 of them MFMA, at a shader clock that falls to 1.7 to 2.0 GHz; at 64
+// reaches 1232 TFLOP/s on this card.) At head dim 128 two chunks of a CU take 4200 cycles of the
+// launch (counters; workgroup starts and ends in it), 2040 of them MFMA on each SIMD, at a
+// shader clock of 1.5 to 1.9 GHz; at 64 (2.2 GHz, MFMA busy 28%)
 // the softmax (32 exponentials, FMAs and packs a chunk) and its issue bound it. Measured
 // and not kept: 256 columns in eight waves (one workgroup per CU at head dim 128, whose
-// start and end, 9 us of 65, nothing then overlaps: 1140 us); the two waves of a SIMD
-// held half a chunk apart by barriers (930 against 911 us on six prompts of 4096); the next
-// chunk's scores computed under this chunk's exponentials (spills at head dim 128); a
+// start and end, 9 us of 65 by marks in a timing copy, nothing then overlaps: 1140 us); the two
+// waves of a SIMD held half a chunk apart by barriers (930 against 911 us on six prompts of 4096);
+// the next chunk's scores computed under this chunk's exponentials (spills at head dim 128); a
 // chunk's loads spread between its products (the same); row sums on the matrix unit (5%
 // slower at head dim 64).
 #include <algorithm>
