@@ -144,8 +144,8 @@ __global__ __launch_bounds__(64 * cshape<D>::NW * SP, 2) void paged_prefill_colu
   const int lane = threadIdx.x & 63, lcol = lane & 31, half = lane >> 5;
   const int4 w0 = a.work[2 * blockIdx.x], w1 = a.work[2 * blockIdx.x + 1];
   const int row0 = w0.x, seq = w0.y, pos0 = w0.z, nrows = w0.w;
+  if (nrows == 0) return;                       // a padding entry (whole workgroup)
   const int col0 = w1.x, kvh = w1.y, part = w1.z, part_chunks = w1.w;
-  if (nrows == 0 || kvh >= a.num_kv_heads) return;   // a padding entry (whole workgroup); a list for other heads
   const int rep = a.rep, ncols = nrows * rep;
 
   // this lane's column: query row my_row of the sequence's new rows, head hd
@@ -462,8 +462,8 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void paged_prefill_columns_f3
   const int lane = threadIdx.x & 63, lcol = lane & 31, half = lane >> 5;
   const int4 w0 = a.work[2 * blockIdx.x], w1 = a.work[2 * blockIdx.x + 1];
   const int row0 = w0.x, seq = w0.y, pos0 = w0.z, nrows = w0.w;
+  if (nrows == 0) return;                       // a padding entry (whole workgroup)
   const int col0 = w1.x, kvh = w1.y, part = w1.z, part_chunks = 2 * w1.w;   // the list counts chunks of 64
-  if (nrows == 0 || kvh >= a.num_kv_heads) return;   // a padding entry (whole workgroup); a list for other heads
   const int rep = a.rep, ncols = nrows * rep;
   const int col = col0 + 32 * wave + lcol;
   const bool mine = col < ncols;
