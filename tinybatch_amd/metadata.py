@@ -113,6 +113,7 @@ class StepMetadata:
     num_columns_work: int = 0
     columns_work: torch.Tensor | None = None
     columns_route: "ColumnsRoute | None" = None
+    columns_heads: tuple | None = None                    # (query, kv) heads of columns_work
     columns_seqs: list | None = None
     columns_partition: int = 0
     columns_other: dict = field(default_factory=dict)
@@ -139,24 +140,20 @@ class StepMetadata:
 
     def columns_list(self, num_heads: int, num_kv_heads: int) -> np.ndarray:
         """The column work list for these heads: columns_work_np for the route's own."""
-        r = self.columns_route
-        if r is None or (r.num_heads, r.num_kv_heads) == (num_heads, num_kv_heads):
+        if self.columns_heads in (None, (num_heads, num_kv_heads)):
             return self.columns_work_np
         return build_columns_work(*zip(*self.columns_seqs), self.columns_partition,
-                                  r._replace(num_heads=num_heads, num_kv_heads=num_kv_heads))
+                                  self.columns_route._replace(num_heads=num_heads, num_kv_heads=num_kv_heads))
 
     def columns_for(self, num_heads: int, num_kv_heads: int, device: torch.device) -> tuple[torch.Tensor, int]:
-        """The uploaded column work list for a call's heads, and its entries. A call with other
-        heads than the route's uploads a list of its own once (not while a graph is captured)."""
-        r = self.columns_route
-        if r is None or (r.num_heads, r.num_kv_heads) == (num_heads, num_kv_heads):
-            return self.columns_work, self.num_columns_work
+        """The column work list of a call with other heads than columns_heads, and its entries:
+        uploaded once (not while a graph is captured)."""
         key = (num_heads, num_kv_heads, device)
         if key not in self.columns_other:
             if torch.cuda.is_current_stream_capturing():
-                raise RuntimeError(f"metadata built for {r.num_heads} / {r.num_kv_heads} heads: a list for {num_heads} "
-                                   f"/ {num_kv_heads} cannot be uploaded while a graph is being captured; call once "
-                                   "before")
+                raise RuntimeError("metadata built for {} / {} heads: ".format(*self.columns_heads) +
+                                   f"a list for {num_heads} / {num_kv_heads} cannot be uploaded while a graph is "
+                                   "being captured; call once before")
             self.columns_other[key] = torch.from_numpy(self.columns_list(num_heads, num_kv_heads)).to(device)
         work = self.columns_other[key]
         return work, int(work.shape[0])
@@ -592,6 +589,7 @@ def build_step_metadata(positions, seq_slices, block_tables, context_lens, *, bl
         columns_work_np=columns_work,
         num_columns_work=0 if columns_work is None else int(columns_work.shape[0]),
         columns_route=None if columns_work is None else columns_route,
+        columns_heads=None if columns_work is None else (columns_route.num_heads, columns_route.num_kv_heads),
         columns_seqs=column_seqs or None,
         columns_partition=columns_part,
         superseded=bool(np.any((slots < 0) & (row_ctx_by_row > 0))),

@@ -597,7 +597,9 @@ def paged_attention(q: torch.Tensor, pool: torch.Tensor, meta: StepMetadata, *, 
             raise ValueError("noalloc takes no workspace")
         if workspace is None and not noalloc:
             workspace = workspace_for(meta, num_heads, d, q.device)
-        columns, num_columns = meta.columns_for(num_heads, hkv, q.device)
+        columns, num_columns = meta.columns_work, meta.num_columns_work
+        if meta.columns_heads not in (None, (num_heads, hkv)):
+            columns, num_columns = meta.columns_for(num_heads, hkv, q.device)
         last = not meta.num_work_items and not meta.num_prefill_tiles
         _lib.check(_lib.lib().tb_paged_prefill_columns(
             q.data_ptr(), qs, pool.data_ptr(), nb, out.data_ptr(), os_, meta.block_tables.data_ptr(),
